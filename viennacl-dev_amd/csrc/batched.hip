@@ -79,12 +79,22 @@ struct BatchDev {
   uint32_t* conv;
 };
 
+// The wavefront sum through shuffles (wave_sum's order).  This kernel is at its register limit, and
+// with the row exchanges of wave_sum the allocator spilled 360 registers more.
+template <typename T>
+__device__ __forceinline__ T batch_wave_sum(T v)
+{
+#pragma unroll
+  for (int o = kWave / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
+  return v;
+}
+
 // Sum over the workgroup of three per-lane values, returned to every lane in a fixed order.
 __device__ __forceinline__ void batch_reduce3(double& a, double& b, double& c, double* red)
 {
-  a = wave_sum(a);
-  b = wave_sum(b);
-  c = wave_sum(c);
+  a = batch_wave_sum(a);
+  b = batch_wave_sum(b);
+  c = batch_wave_sum(c);
   const int wave = threadIdx.x / kWave;
   if ((threadIdx.x & (kWave - 1)) == 0) {
     red[wave * 3 + 0] = a;
@@ -237,7 +247,7 @@ __device__ __forceinline__ void batch_spmv_staged(const BatchDev<T>& B, uint32_t
           const uint32_t z = min(srp[row + 1], cnt);
           T sum = 0;
           for (uint32_t k = min(srp[row], z) + lane; k < z; k += kWave) sum += stage[k];
-          sum = wave_sum(sum);
+          sum = batch_wave_sum(sum);
           if (lane == 0) {
             const uint32_t li = r0 - rs + row;
             ap[li] = sum;

@@ -29,12 +29,86 @@ __device__ __forceinline__ void keep_here(T& v)
   asm volatile("" : "+v"(v));
 }
 
+// The value of the lane whose index differs in one bit, for the five exchanges below.  They run in the
+// vector pipeline (row rotations, quad permutes and gfx950's half- and row-swaps), where __shfl_xor
+// goes through LDS: a wavefront sum of a double takes 6 exchanges, each about 100 cycles of latency
+// there and about 10 here.
+template <int Ctrl, typename T>
+__device__ __forceinline__ T dpp_move(T v)
+{
+  if constexpr (sizeof(T) == 8) {
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+    const int l = static_cast<int>(u), h = static_cast<int>(u >> 32);
+    const uint32_t l2 = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(l, l, Ctrl, 0xf, 0xf, false));
+    const uint32_t h2 = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(h, h, Ctrl, 0xf, 0xf, false));
+    return __builtin_bit_cast(T, static_cast<unsigned long long>(h2) << 32 | l2);
+  } else {
+    const int l = __builtin_bit_cast(int, v);
+    return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(l, l, Ctrl, 0xf, 0xf, false));
+  }
+}
+
+// Exchanges 32-lane halves (Rows = 32) or 16-lane rows (16) between a and b: afterwards a holds the
+// even halves (rows) of both and b the odd ones, so that a + b adds each value's own two halves
+// (rows), a's in the even and b's in the odd ones.
+template <int Rows, typename T>
+__device__ __forceinline__ void swap_rows(T& a, T& b)
+{
+  auto swap32 = [](uint32_t& x, uint32_t& y) {
+    if constexpr (Rows == 32) {
+      const auto r = __builtin_amdgcn_permlane32_swap(x, y, false, false);
+      x = r[0];
+      y = r[1];
+    } else {
+      const auto r = __builtin_amdgcn_permlane16_swap(x, y, false, false);
+      x = r[0];
+      y = r[1];
+    }
+  };
+  if constexpr (sizeof(T) == 8) {
+    const unsigned long long ua = __builtin_bit_cast(unsigned long long, a), ub = __builtin_bit_cast(unsigned long long, b);
+    uint32_t al = static_cast<uint32_t>(ua), ah = static_cast<uint32_t>(ua >> 32);
+    uint32_t bl = static_cast<uint32_t>(ub), bh = static_cast<uint32_t>(ub >> 32);
+    swap32(al, bl);
+    swap32(ah, bh);
+    a = __builtin_bit_cast(T, static_cast<unsigned long long>(ah) << 32 | al);
+    b = __builtin_bit_cast(T, static_cast<unsigned long long>(bh) << 32 | bl);
+  } else {
+    uint32_t x = __builtin_bit_cast(uint32_t, a), y = __builtin_bit_cast(uint32_t, b);
+    swap32(x, y);
+    a = __builtin_bit_cast(T, x);
+    b = __builtin_bit_cast(T, y);
+  }
+}
+
+constexpr int kDppXor1 = 0xB1;   // quad_perm [1, 0, 3, 2]
+constexpr int kDppXor2 = 0x4E;   // quad_perm [2, 3, 0, 1]
+constexpr int kDppRor4 = 0x124;  // row_ror:4 -- lane ^ 4 where the values repeat every eight lanes
+constexpr int kDppRor8 = 0x128;  // row_ror:8 -- lane ^ 8
+
+// The last four steps of the wavefront sum: over each 16-lane row, in the order 8, 4, 2, 1.
+template <typename T>
+__device__ __forceinline__ T row_sum(T v)
+{
+  v += dpp_move<kDppRor8>(v);
+  v += dpp_move<kDppRor4>(v);
+  v += dpp_move<kDppXor2>(v);
+  v += dpp_move<kDppXor1>(v);
+  return v;
+}
+
+// Sum over the wavefront, returned to every lane: the xor butterfly 32, 16, 8, 4, 2, 1.
 template <typename T>
 __device__ __forceinline__ T wave_sum(T v)
 {
-#pragma unroll
-  for (int o = kWave / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
-  return v;
+  static_assert(sizeof(T) == 8 || sizeof(T) == 4);
+  T u = v;
+  swap_rows<32>(v, u);
+  v += u;
+  u = v;
+  swap_rows<16>(v, u);
+  v += u;
+  return row_sum(v);
 }
 
 // Sum over aligned groups of L lanes (L a power of two <= 64).

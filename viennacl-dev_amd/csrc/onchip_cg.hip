@@ -1,0 +1,790 @@
+// onchip_cg.hip -- all CG iterations of a DIA system in one launch, the vectors held on chip.
+//
+// A kernel per step reads and writes every vector through the memory side of the chip in every
+// iteration (seven passes in the update, two in the product) and pays a kernel boundary per step.
+// The register files (512 KB a CU, 128 MB in all) hold the whole solve instead: a workgroup of 1024
+// lanes per CU owns a contiguous range of rows (the owners of cg_sums.hpp) with x, r and A p in
+// registers and p in LDS, and runs every iteration on them.  Between CUs travel
+//   * the inner products: a workgroup publishes its three sums in one 64-byte line, each double as
+//     two 8-byte words that carry the iteration number, and every workgroup reads all lines until
+//     the numbers are right.  Data and flag are one word, so no order between stores is needed, and
+//     the lines alternate between two sets, so that none is overwritten before everyone has read it;
+//   * the rows of p that the stencil reaches outside a workgroup's own range.  Two forms:
+//     ghost: the workgroup keeps r and p of those rows as well (r in registers, p in LDS) and
+//       updates them itself from its neighbours' A p, which they stored before they published their
+//       sums: one exchange per iteration;
+//     halo:  p of the own rows is stored after the update, neighbours are told by a flag, and the
+//       reached rows are read from memory: a second, neighbours-only wait per iteration, but no
+//       ghost state, for systems whose ghost rows would not fit.
+// Data that another workgroup reads is stored and loaded at agent scope (past the XCD's L2, which is
+// not coherent with the others), and a wave waits for its stores before its workgroup publishes.
+// The operator's values stay in registers (small systems), or as packed 4-bit codes into value
+// tables in LDS, or are read again in every iteration (they then come from the caches).
+//
+// Every sum is formed in the order of the kernel-per-step modes (cg_sums.hpp), so the results are
+// theirs bit for bit.
+//
+// All workgroups must run at once.  The grid is at most one workgroup per CU and one on-chip solve
+// per device runs at a time (a host lock); every wait is bounded by the wall clock, and a workgroup
+// that gives up raises a flag that ends all the others' waits.
+#include <algorithm>
+#include <cstdlib>
+#include <mutex>
+
+#include "cg_sums.hpp"
+#include "internal.hpp"
+#include "onchip_cg.hpp"
+
+namespace vclhip {
+
+// Measurement and test hooks (vclhip_onchip_*), per thread.
+static thread_local double t_wait_us = -1;
+static thread_local int t_on_chip = 0;
+
+namespace {
+
+constexpr int kOcThreads = 1024;
+constexpr int kOcBlocks = kOcThreads / kBlock;  // 256-lane groups of a workgroup, one chunk at a time each
+constexpr uint32_t kOcDiags = 8;                // diagonals at most
+constexpr uint32_t kOcChunks = 8;               // chunks of a workgroup at most
+constexpr int kOcSums = 3;
+constexpr uint32_t kOcLine = 8;                 // 8-byte words of a workgroup's line
+constexpr size_t kOcLds = 160 * 1024 - 2048;    // dynamic LDS at most (the static part stays below 2 KB)
+constexpr uint64_t kOcClock = 100;              // wall clock ticks per microsecond
+
+enum OcVal { kValRegs = 0, kValCodes = 1, kValStream = 2 };
+
+// Relaxed accesses at agent scope: single-location coherence between the XCDs.
+template <typename U>
+__device__ __forceinline__ U ld_agent(const U* p)
+{
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename U>
+__device__ __forceinline__ void st_agent(U* p, U v)
+{
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// A device array as a buffer resource: 32-bit byte offsets instead of 64-bit addresses, loads past
+// its end give 0 and stores past it do nothing.  Agent: at agent scope, as above.
+template <typename T>
+struct OcBuf {
+  __amdgpu_buffer_rsrc_t rsrc;
+  __device__ __forceinline__ OcBuf(const T* p, size_t count)
+      : rsrc(__builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(p), 0, static_cast<int>(count * sizeof(T)), 0x00027000))
+  {
+  }
+  template <bool Agent = false>
+  __device__ __forceinline__ T load(uint32_t i) const
+  {
+    constexpr int aux = Agent ? 16 : 0;
+    if constexpr (sizeof(T) == 8)
+      return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(rsrc, i * sizeof(T), 0, aux));
+    else if constexpr (sizeof(T) == 4)
+      return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(rsrc, i * sizeof(T), 0, aux));
+    else
+      return __builtin_amdgcn_raw_buffer_load_b8(rsrc, i, 0, aux);
+  }
+  template <bool Agent = false>
+  __device__ __forceinline__ void store(uint32_t i, T v) const
+  {
+    constexpr int aux = Agent ? 16 : 0;
+    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+    if constexpr (sizeof(T) == 8)
+      __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), rsrc, i * sizeof(T), 0, aux);
+    else
+      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), rsrc, i * sizeof(T), 0, aux);
+  }
+};
+constexpr uint32_t kOcNowhere = 0x1ffffff0u;  // an index past the end of every buffer
+
+// The rows that a workgroup of `rows` rows reaches along its diagonals, as disjoint segments in LDS
+// one after the other: its row l (counted from its first) is entry own + l, and that row's neighbour
+// on diagonal i entry delta[i] + l.  Rows outside the system have entries too (they stay zero), so
+// that no access needs a check.  Diagonals of `far` are left out.  Offsets ascending.
+struct OcSegments {
+  uint32_t count, ext, own;
+  int32_t start[kOcDiags + 1];  // first row of the segment, from the workgroup's first row
+  uint32_t base[kOcDiags + 1];  // its entry
+  uint32_t delta[kOcDiags];
+};
+
+__host__ __device__ inline void oc_segments(uint32_t rows, uint32_t nd, const int32_t* off, uint32_t far, OcSegments& g)
+{
+  g.count = 0;
+  g.ext = 0;
+  g.own = 0;
+  int32_t end = 0;
+  bool own_done = false;
+  for (uint32_t i = 0; i <= nd; ++i) {
+    for (int pass = 0; pass < 2; ++pass) {
+      // pass 0: the own rows, in front of the first diagonal at or above 0; pass 1: diagonal i
+      if (pass == 0 ? own_done || (i < nd && off[i] < 0) : i == nd || (far >> i & 1u) != 0) continue;
+      const int32_t s = pass == 0 ? 0 : off[i], e = s + static_cast<int32_t>(rows);
+      own_done = own_done || pass == 0;
+      if (g.count == 0 || s > end) {
+        g.start[g.count] = s;
+        g.base[g.count] = g.ext;
+        ++g.count;
+        end = s;
+      }
+      g.ext += static_cast<uint32_t>(e - end);
+      end = e;
+      const uint32_t at = g.base[g.count - 1] + static_cast<uint32_t>(s - g.start[g.count - 1]);
+      if (pass == 0)
+        g.own = at;
+      else
+        g.delta[i] = at;
+    }
+  }
+}
+
+// Workgroup w's owners, product chunks and tiles.
+struct OcPart {
+  uint32_t o0, o1, p0, p1, t0, t1;
+};
+
+__host__ __device__ inline OcPart oc_part(uint32_t n, uint32_t gp, uint32_t m, uint32_t w)
+{
+  OcPart q;
+  const uint32_t tiles = cg_tiles(n), owners = gp < kOwners ? gp : kOwners;
+  q.o0 = w * m;
+  q.o1 = q.o0 + m < owners ? q.o0 + m : owners;
+  uint32_t unused;
+  owner_range(gp, q.o0, q.p0, unused);
+  owner_range(gp, q.o1 - 1, unused, q.p1);
+  part_range(tiles, q.p0, gp, q.t0, unused);
+  part_range(tiles, q.p1, gp, q.t1, unused);
+  return q;
+}
+
+template <typename T>
+struct OcArgs {
+  uint32_t n, nd, gp, m, nwg;
+  uint32_t far;     // halo form: mask of the diagonals read from memory (at most two)
+  uint32_t ext;     // LDS entries for p
+  uint32_t reach;   // halo form: workgroups on each side that own reached rows
+  int32_t off[kOcDiags];
+  const T* val;
+  const uint8_t* code;
+  const T* table;
+  T* x;
+  const T* r;
+  const T* p;
+  const T* d;
+  T* ex0;  // ghost form: A p of even iterations; halo form: p
+  T* ex1;  // ghost form: A p of odd iterations, and of the first direction
+  KState* st;
+  unsigned long long* lines;  // two sets of one line per workgroup
+  uint32_t* flags;            // halo form: one 64-byte line per workgroup
+  uint32_t* abort;
+  uint64_t wait;              // wall clock ticks that a wait may take
+};
+
+// One poll more after a failed one?  Looks at the abort flag and the clock now and then (always
+// when the limit is zero, which is how a test makes a wait give up).
+struct OcWait {
+  uint64_t t0 = 0;  // read at the first look
+  uint32_t polls = 0;
+  __device__ __forceinline__ bool again(uint32_t* abort, uint64_t limit)
+  {
+    if ((++polls & 63u) != 0 && limit != 0) return true;
+    const uint64_t now = wall_clock64();
+    if (t0 == 0) t0 = now;
+    if (ld_agent(abort) == 0 && now - t0 < limit) return true;
+    st_agent(abort, 1u);
+    return false;
+  }
+};
+
+// W: the width of the vector kernels' packs.  CPV: chunks of a 256-lane group at most, TPC:
+// tiles of a chunk at most (CPV * TPC rows a lane).  Ghosts: ghost rows a lane at most, 0 for the
+// halo form.
+template <typename T, bool Jac, int W, int CPV, int TPC, OcVal Val, int Ghosts>
+__global__ __launch_bounds__(kOcThreads) void onchip_cg_kernel(OcArgs<T> a)
+{
+  constexpr int S = CPV * TPC;
+  extern __shared__ __align__(16) unsigned char oc_lds[];
+  __shared__ double red[kOcSums][kOcChunks][kWavesPerBlock];
+  __shared__ double tot[kOcSums][kWavesPerBlock];
+  __shared__ OcSegments seg;
+  __shared__ uint32_t ok;
+
+  KState* const st = a.st;
+  if (st->flags & kFlagDone) return;
+  const uint32_t tid = threadIdx.x, w = blockIdx.x, n = a.n, nd = a.nd;
+  const uint32_t vb = __builtin_amdgcn_readfirstlane(tid / kBlock), t = tid % kBlock;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane((tid / kWave) % kWavesPerBlock), lane = tid % kWave;
+  const OcPart q = oc_part(n, a.gp, a.m, w);
+  const uint32_t lo = q.t0 * kBlock, rows = (q.t1 - q.t0) * kBlock;  // rows past the system's end are held as zeros
+  const uint32_t mv = a.gp <= kOwners ? 1u : cg_vec_per_owner(n);
+  const uint32_t v0 = a.gp <= kOwners ? q.o0 : q.o0 * mv;
+  const uint32_t nvec = (q.o1 - q.o0) * mv, nprod = q.p1 - q.p0;
+
+  T* const stab = reinterpret_cast<T*>(oc_lds);
+  T* const lp = stab + (Val == kValCodes ? kOcDiags * kDiaCodes : 0u);
+  T* const lsq = lp + a.ext;
+
+  if (tid == 0) {
+    ok = 1;
+    oc_segments(rows, nd, a.off, a.far, seg);
+  }
+  if constexpr (Val == kValCodes)
+    for (uint32_t i = tid; i < nd * kDiaCodes; i += kOcThreads) stab[i] = a.table[i];
+  for (uint32_t i = tid; i < a.ext; i += kOcThreads) lp[i] = T(0);
+  __syncthreads();
+  uint32_t delta[kOcDiags];
+#pragma unroll
+  for (uint32_t i = 0; i < kOcDiags; ++i)
+    delta[i] = i < nd && !(a.far >> i & 1u) ? __builtin_amdgcn_readfirstlane(seg.delta[i]) : 0u;
+  const uint32_t own = __builtin_amdgcn_readfirstlane(seg.own);
+  const uint32_t ghosts = __builtin_amdgcn_readfirstlane(seg.ext) - rows;
+
+  const OcBuf<T> bval(a.val, static_cast<size_t>(nd) * n), bx(a.x, n), br(a.r, n), bp(a.p, n), bd(Jac ? a.d : a.r, n);
+  const OcBuf<T> bex0(a.ex0, n), bex1(a.ex1, n);
+  const OcBuf<uint8_t> bcode(a.code, a.code ? static_cast<size_t>(nd) * n : 0);
+
+  // the lane's rows: tile j of chunk c is the workgroup's row first[c] + j * kBlock, for j < cnt[c]
+  uint32_t first[CPV], cnt[CPV];
+#pragma unroll
+  for (int c = 0; c < CPV; ++c) {
+    const uint32_t pc = q.p0 + vb + static_cast<uint32_t>(c) * kOcBlocks;
+    uint32_t b = q.t0, e = q.t0;
+    if (pc < q.p1) part_range(cg_tiles(n), pc, a.gp, b, e);
+    first[c] = (b - q.t0) * kBlock + t;
+    cnt[c] = __builtin_amdgcn_readfirstlane(e - b);
+  }
+  // the vector chunks, as rows of the workgroup
+  uint32_t vc0[CPV], vc1[CPV];
+#pragma unroll
+  for (int c = 0; c < CPV; ++c) {
+    const uint32_t vc = vb + static_cast<uint32_t>(c) * kOcBlocks;
+    uint32_t b = lo, e = lo;
+    if (vc < nvec) cg_vec_rows(n, v0 + vc, b, e);
+    vc0[c] = __builtin_amdgcn_readfirstlane(b - lo);
+    vc1[c] = __builtin_amdgcn_readfirstlane(e - lo);
+  }
+
+  T x[S], r[S], ap[S];
+  T v[Val == kValRegs ? S : 1][kOcDiags];
+  uint32_t codes[Val == kValCodes ? S : 1];
+#pragma unroll
+  for (int c = 0; c < CPV; ++c)
+#pragma unroll
+    for (int j = 0; j < TPC; ++j) {
+      const int s = c * TPC + j;
+      x[s] = r[s] = ap[s] = T(0);
+      if constexpr (Val == kValRegs)
+#pragma unroll
+        for (uint32_t i = 0; i < kOcDiags; ++i) v[s][i] = T(0);
+      if constexpr (Val == kValCodes) codes[s] = 0;
+      if (static_cast<uint32_t>(j) < cnt[c]) {
+        const uint32_t l = first[c] + j * kBlock, row = lo + l;
+        r[s] = br.load(row);
+        ap[s] = bex1.load(row);
+        lp[own + l] = bp.load(row);
+#pragma unroll
+        for (uint32_t i = 0; i < kOcDiags; ++i)
+          if (i < nd && row < n) {
+            if constexpr (Val == kValRegs)
+              v[s][i] = a.code ? a.table[i * kDiaCodes + bcode.load(i * n + row)] : bval.load(i * n + row);
+            if constexpr (Val == kValCodes) codes[s] |= static_cast<uint32_t>(bcode.load(i * n + row)) << (4 * i);
+          }
+      }
+    }
+
+  // the lane's ghost rows: LDS entries tid, tid + 1024, ... of the entries beside the own rows
+  constexpr int NG = Ghosts > 0 ? Ghosts : 1;
+  uint32_t grow[NG];
+  T gr[NG];
+  auto ghost_at = [&](uint32_t g) { return g < own ? g : g + rows; };
+  auto ghost_row = [&](uint32_t e) {  // kOcNowhere outside the system
+    uint32_t k = 0;
+    while (k + 1 < seg.count && e >= seg.base[k + 1]) ++k;
+    const uint32_t row = lo + static_cast<uint32_t>(seg.start[k]) + (e - seg.base[k]);
+    return row < n ? row : kOcNowhere;
+  };
+  if constexpr (Ghosts > 0) {
+#pragma unroll
+    for (int k = 0; k < NG; ++k) {
+      const uint32_t g = tid + static_cast<uint32_t>(k) * kOcThreads;
+      grow[k] = kOcNowhere;
+      gr[k] = T(0);
+      if (g < ghosts) {
+        const uint32_t e = ghost_at(g);
+        grow[k] = ghost_row(e);
+        gr[k] = br.load(grow[k]);
+        lp[e] = bp.load(grow[k]);
+      }
+    }
+  }
+
+  // wave 0 reduces the chunk partials: lane 8 q + ch holds chunk ch of sum q, lane 8 q + o owner o
+  const uint32_t rq = lane >> 3, rc = lane & 7u;
+  uint32_t own_b = 0, own_e = 0;
+  if (rc < q.o1 - q.o0) {
+    if (rq == 0) {
+      own_b = rc * mv;
+      own_e = own_b + mv;
+    } else {
+      owner_range(a.gp, q.o0 + rc, own_b, own_e);
+      own_b -= q.p0;
+      own_e -= q.p0;
+    }
+  }
+
+  const double nrs = st->nrs, tol2 = st->tol * st->tol, atol2 = st->abs_tol * st->abs_tol;
+  const uint32_t max_iters = st->max_iters;
+  double alpha = st->alpha, beta = st->beta;
+  const __amdgpu_buffer_rsrc_t line_rsrc =
+      __builtin_amdgcn_make_buffer_rsrc(a.lines, 0, 2 * kOwners * kOcLine * 8, 0x00027000);
+
+  for (uint32_t k = 0;; ++k) {
+    // nothing derived from a lane's rows is kept across iterations: it is cheaper to form again than
+    // to spill
+#pragma unroll
+    for (int c = 0; c < CPV; ++c) keep_here(first[c]);
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      if constexpr (Val == kValCodes) keep_here(codes[s]);
+      if constexpr (Val == kValRegs)
+#pragma unroll
+        for (uint32_t i = 0; i < kOcDiags; ++i) keep_here(v[s][i]);
+    }
+    // ---- update: x, r, p of the own rows (and r, p of the ghosts from the neighbours' A p)
+    const T ta = static_cast<T>(alpha), tb = static_cast<T>(beta);
+    const OcBuf<T>& ex_in = Ghosts > 0 && !(k & 1u) ? bex1 : bex0;
+    const OcBuf<T>& ex_out = Ghosts > 0 && (k & 1u) ? bex1 : bex0;
+    T ga[NG], gd[NG];
+    if constexpr (Ghosts > 0) {
+#pragma unroll
+      for (int i = 0; i < NG; ++i) {
+        if (static_cast<uint32_t>(i) * kOcThreads < ghosts) {
+          ga[i] = ex_in.template load<true>(grow[i]);
+          if constexpr (Jac) gd[i] = bd.load(grow[i]);
+        }
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < CPV; ++c)
+#pragma unroll
+      for (int j = 0; j < TPC; ++j)
+        if (static_cast<uint32_t>(j) < cnt[c]) {
+          const int s = c * TPC + j;
+          const uint32_t l = first[c] + j * kBlock;
+          T pv = lp[own + l];
+          x[s] += ta * pv;
+          r[s] -= ta * ap[s];
+          T z = r[s];
+          if constexpr (Jac) z = lo + l < n ? r[s] / bd.load(lo + l) : T(0);
+          pv = z + tb * pv;
+          lp[own + l] = pv;
+          lsq[l] = r[s] * z;
+          if constexpr (Ghosts == 0) ex_out.template store<true>(lo + l, pv);
+        }
+    if constexpr (Ghosts > 0) {
+#pragma unroll
+      for (int i = 0; i < NG; ++i) {
+        const uint32_t g = tid + static_cast<uint32_t>(i) * kOcThreads;
+        if (g < ghosts) {
+          const uint32_t e = ghost_at(g);
+          gr[i] -= ta * ga[i];
+          T z = gr[i];
+          if constexpr (Jac) z = gr[i] / gd[i];
+          lp[e] = z + tb * lp[e];
+        }
+      }
+    } else {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // p is where the neighbours read it
+    }
+    __syncthreads();
+    if constexpr (Ghosts == 0) {
+      if (tid == 0) st_agent(a.flags + w * 16, k + 1);
+    }
+
+    // ---- partial sums of <r,z> per vector chunk, in the packs' order
+    double acc_v[CPV];
+#pragma unroll
+    for (int c = 0; c < CPV; ++c) {
+      acc_v[c] = 0;
+      const uint32_t packed_end = vc0[c] + ((vc1[c] - vc0[c]) / W) * W;
+      for (uint32_t i = vc0[c] + W * t; i < packed_end; i += W * kBlock)
+#pragma unroll
+        for (int e = 0; e < W; ++e) acc_v[c] += static_cast<double>(lsq[i + e]);
+      if (W > 1)
+        for (uint32_t i = packed_end + t; i < vc1[c]; i += kBlock) acc_v[c] += static_cast<double>(lsq[i]);
+    }
+
+    // ---- halo form: wait for the neighbours' p, then read what the stencil reaches
+    T far0[S], far1[S];
+    uint32_t f0 = 0, f1 = 0;
+    if constexpr (Ghosts == 0) {
+      if (tid >= kOcThreads - 2 * kWave) {
+        const uint32_t i = tid - (kOcThreads - 2 * kWave);
+        if (i <= 2 * a.reach && w + i >= a.reach && w + i - a.reach < a.nwg) {
+          OcWait wait;
+          while (ld_agent(a.flags + (w + i - a.reach) * 16) < k + 1)
+            if (!wait.again(a.abort, a.wait)) {
+              ok = 0;
+              break;
+            }
+        }
+      }
+      __syncthreads();
+      if (!ok) return;
+      f0 = a.far ? static_cast<uint32_t>(__builtin_ctz(a.far)) : kOcDiags;
+      f1 = a.far & (a.far - 1) ? static_cast<uint32_t>(__builtin_ctz(a.far & (a.far - 1))) : kOcDiags;
+#pragma unroll
+      for (int c = 0; c < CPV; ++c)
+#pragma unroll
+        for (int j = 0; j < TPC; ++j) {
+          const int s = c * TPC + j;
+          if (static_cast<uint32_t>(j) < cnt[c]) {
+            const uint32_t row = lo + first[c] + j * kBlock;
+            if (f0 < kOcDiags) {
+              const uint32_t cc = row + static_cast<uint32_t>(a.off[f0]);
+              far0[s] = ex_in.template load<true>(cc < n ? cc : kOcNowhere);
+            }
+            if (f1 < kOcDiags) {
+              const uint32_t cc = row + static_cast<uint32_t>(a.off[f1]);
+              far1[s] = ex_in.template load<true>(cc < n ? cc : kOcNowhere);
+            }
+          }
+        }
+      for (uint32_t g = tid; g < ghosts; g += kOcThreads) {
+        const uint32_t e = ghost_at(g);
+        lp[e] = ex_in.template load<true>(ghost_row(e));
+      }
+      __syncthreads();
+    }
+
+    // ---- product: A p of the own rows (dia_kernel's sum), <Ap,Ap> and <p,Ap> per product chunk
+    double acc_a[CPV], acc_p[CPV];
+#pragma unroll
+    for (int c = 0; c < CPV; ++c) {
+      acc_a[c] = acc_p[c] = 0;
+#pragma unroll
+      for (int j = 0; j < TPC; ++j)
+        if (static_cast<uint32_t>(j) < cnt[c]) {
+          const int s = c * TPC + j;
+          const uint32_t l = first[c] + j * kBlock, row = lo + l;
+          T vv[kOcDiags];
+          if constexpr (Val == kValStream)
+#pragma unroll
+            for (uint32_t i = 0; i < kOcDiags; ++i)
+              if (i < nd) vv[i] = bval.load(row < n ? i * n + row : kOcNowhere);
+          T sum = 0;
+#pragma unroll
+          for (uint32_t i = 0; i < kOcDiags; ++i)
+            if (i < nd) {
+              T xv;
+              if (Ghosts == 0 && i == f0)
+                xv = far0[s];
+              else if (Ghosts == 0 && i == f1)
+                xv = far1[s];
+              else
+                xv = lp[delta[i] + l];
+              T val;
+              if constexpr (Val == kValRegs) val = v[s][i];
+              if constexpr (Val == kValCodes) val = stab[i * kDiaCodes + (codes[s] >> (4 * i) & 15u)];
+              if constexpr (Val == kValStream) val = vv[i];
+              sum += (val > 0 || val < 0) ? xv * val : T(0);
+            }
+          ap[s] = sum;
+          if constexpr (Ghosts > 0) ex_out.template store<true>(row, sum);
+          if constexpr (Jac)
+            acc_a[c] += static_cast<double>(row < n ? sum * (sum / bd.load(row)) : T(0));
+          else
+            acc_a[c] += static_cast<double>(sum * sum);
+          acc_p[c] += static_cast<double>(lp[own + l] * sum);
+        }
+    }
+
+    // ---- the workgroup's three sums
+#pragma unroll
+    for (int c = 0; c < CPV; ++c) {
+      const uint32_t at = vb + static_cast<uint32_t>(c) * kOcBlocks;
+      const double sv = wave_sum(acc_v[c]), sa = wave_sum(acc_a[c]), sp = wave_sum(acc_p[c]);
+      if (lane == 0) {
+        red[0][at][wave] = sv;
+        red[1][at][wave] = sa;
+        red[2][at][wave] = sp;
+      }
+    }
+    if constexpr (Ghosts > 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // A p is where the neighbours read it
+    __syncthreads();
+    unsigned long long* const set = a.lines + (k & 1u) * kOwners * kOcLine;
+    if (tid < kWave) {
+      double part = 0;
+      if (rq < kOcSums && rc < (rq == 0 ? nvec : nprod)) {
+        part = red[rq][rc][0];
+#pragma unroll
+        for (int i = 1; i < kWavesPerBlock; ++i) part += red[rq][rc][i];
+      }
+      double sum = 0;
+#pragma unroll
+      for (uint32_t i = 0; i < CPV * kOcBlocks; ++i) {
+        const double u = __shfl(part, static_cast<int>((rq << 3) + ((own_b + i) & 7u)), kWave);
+        if (own_b + i < own_e) sum += u;
+      }
+      if (a.m >= 2) sum += __shfl_xor(sum, 1, kWave);
+      if (a.m >= 4) sum += __shfl_xor(sum, 2, kWave);
+      sum = __shfl(sum, static_cast<int>(((lane >> 1) & 7u) << 3), kWave);
+      if (lane < 2 * kOcSums) {
+        const unsigned long long bits = static_cast<unsigned long long>(__double_as_longlong(sum));
+        const unsigned long long half = (lane & 1u) ? bits >> 32 : bits & 0xffffffffull;
+        st_agent(set + w * kOcLine + lane, static_cast<unsigned long long>(k + 1) << 32 | half);
+      }
+    }
+    // ---- everyone's sums, then the binary tree over them
+    if (tid < kOwners) {
+      double s3[kOcSums] = {0, 0, 0};
+      if (tid < a.nwg) {
+        OcWait wait;
+        uint32_t word[4 * kOcSums];
+        for (;;) {
+          bool all = true;
+#pragma unroll
+          for (int i = 0; i < kOcSums; ++i) {
+            typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+            const u32x4 b = __builtin_amdgcn_raw_buffer_load_b128(
+                line_rsrc, ((k & 1u) * kOwners + tid) * kOcLine * 8 + 16 * i, 0, 16);
+            word[4 * i] = b.x;
+            word[4 * i + 1] = b.y;
+            word[4 * i + 2] = b.z;
+            word[4 * i + 3] = b.w;
+          }
+          asm volatile("" ::: "memory");
+#pragma unroll
+          for (int i = 0; i < 2 * kOcSums; ++i) all = all && word[2 * i + 1] == k + 1;
+          if (all) break;
+          if (!wait.again(a.abort, a.wait)) {
+            ok = 0;
+            break;
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < kOcSums; ++i)
+          s3[i] = __longlong_as_double(static_cast<long long>(static_cast<unsigned long long>(word[4 * i + 2]) << 32 | word[4 * i]));
+      }
+#pragma unroll
+      for (int i = 0; i < kOcSums; ++i) {
+#pragma unroll
+        for (int o = 1; o < kWave; o <<= 1) s3[i] += __shfl_xor(s3[i], o, kWave);
+        if (lane == 0) tot[i][wave] = s3[i];
+      }
+    }
+    __syncthreads();
+    if (!ok) return;
+    const double rr = (tot[0][0] + tot[0][1]) + (tot[0][2] + tot[0][3]);
+    const double ApAp = (tot[1][0] + tot[1][1]) + (tot[1][2] + tot[1][3]);
+    const double pAp = (tot[2][0] + tot[2][1]) + (tot[2][2] + tot[2][3]);
+
+    // ---- cg_iter_kernel's step (cg.hpp:170-180)
+    const uint32_t iter = k + 1;
+    const bool conv = fabs(rr / nrs) < tol2 || fabs(rr) < atol2;
+    const bool done = conv || iter >= max_iters;
+    if (w == 0 && tid == 0) {
+      record_history(st, iter, rr);
+      if (done) {
+        st->iter = iter;
+        st->rr = rr;
+        st->converged = conv ? 1u : 0u;
+        st->flags |= kFlagDone;
+      }
+    }
+    if (done) break;
+    alpha = rr / pAp;
+    beta = (alpha * alpha * ApAp - rr) / rr;
+  }
+
+#pragma unroll
+  for (int c = 0; c < CPV; ++c)
+#pragma unroll
+    for (int j = 0; j < TPC; ++j)
+      if (static_cast<uint32_t>(j) < cnt[c]) bx.store(lo + first[c] + j * kBlock, x[c * TPC + j]);
+}
+
+// ------------------------------------------------------------------ host side
+
+// One on-chip solve per device at a time: a second one takes the other modes instead of waiting.
+std::mutex g_slot[64];
+
+uint64_t wait_ticks()
+{
+  return t_wait_us < 0 ? 500000 * kOcClock : static_cast<uint64_t>(t_wait_us * kOcClock);
+}
+
+// The shape of an on-chip solve and the kernel that runs it.
+template <typename T>
+struct OcPlan {
+  void (*kernel)(OcArgs<T>) = nullptr;
+  uint32_t m = 0, nwg = 0, ext = 0, far = 0, reach = 0;
+  bool ghost = false;
+  size_t lds = 0;
+};
+
+template <typename T, bool Jac, int W>
+void (*oc_kernel(bool ghost, int cpv, int tpc, uint32_t ghosts, bool coded))(OcArgs<T>)
+{
+  constexpr uint32_t g1 = kOcThreads;
+  if (ghost) {
+    // up to two rows a lane: the values in registers; four: codes or a stream
+    if (cpv == 1 && tpc == 1 && ghosts <= 6 * g1) return onchip_cg_kernel<T, Jac, W, 1, 1, kValRegs, 6>;
+    if (cpv <= 2 && tpc == 1 && ghosts <= 6 * g1) return onchip_cg_kernel<T, Jac, W, 2, 1, kValRegs, 6>;
+    if (cpv <= 2 && tpc <= 2 && ghosts <= 9 * g1)
+      return coded ? onchip_cg_kernel<T, Jac, W, 2, 2, kValCodes, 9> : onchip_cg_kernel<T, Jac, W, 2, 2, kValStream, 9>;
+    return nullptr;
+  }
+  if (cpv <= 2 && tpc <= 2)
+    return coded ? onchip_cg_kernel<T, Jac, W, 2, 2, kValCodes, 0> : onchip_cg_kernel<T, Jac, W, 2, 2, kValStream, 0>;
+  if (cpv <= 2 && tpc <= 4)
+    return coded ? onchip_cg_kernel<T, Jac, W, 2, 4, kValCodes, 0> : onchip_cg_kernel<T, Jac, W, 2, 4, kValStream, 0>;
+  return nullptr;
+}
+
+template <typename T>
+bool oc_plan(const OnchipCg<T>& c, OcPlan<T>& pl)
+{
+  const uint32_t n = c.n, nd = c.dia.nd;
+  if (!c.off_host || nd == 0 || nd > kOcDiags || n >= (1u << 24)) return false;  // 32-bit byte offsets
+  const uint32_t gp = cg_prod_chunks(n), tiles = cg_tiles(n);
+  const uint32_t owners = gp < kOwners ? gp : kOwners;
+  // fewer workgroups exchange faster (2.3 us for 64, 2.4 for 128, 2.8 for 256), so small systems put
+  // several owners, one chunk or two each, on a workgroup's four 256-lane groups
+  pl.m = gp <= kOwners ? 4u : (gp <= 2 * kOwners ? 2u : 1u);
+  pl.nwg = (owners + pl.m - 1) / pl.m;
+  if (pl.nwg > static_cast<uint32_t>(device_cu_count())) return false;
+  const uint32_t chunks = pl.m * ((gp + kOwners - 1) / kOwners);  // of a workgroup, at most
+  const uint32_t vecs = pl.m * (gp <= kOwners ? 1u : cg_vec_per_owner(n));
+  const int cpv = static_cast<int>((std::max(chunks, vecs) + kOcBlocks - 1) / kOcBlocks);
+  const int tpc = static_cast<int>((tiles + gp - 1) / gp);
+  auto wg_tiles = [&](bool up) { return static_cast<uint32_t>((static_cast<uint64_t>(tiles) * chunks + (up ? gp - 1 : 0)) / gp); };
+  const uint32_t rows = wg_tiles(true) * kBlock;
+  const size_t tab = c.dia.code ? kOcDiags * kDiaCodes * sizeof(T) : 0;
+  int32_t reach_rows = 0;
+  for (uint32_t i = 0; i < nd; ++i) reach_rows = std::max(reach_rows, std::abs(c.off_host[i]));
+  // the LDS entries of a full workgroup: no workgroup has more
+  auto segments = [&](uint32_t far) {
+    OcSegments g;
+    oc_segments(rows, nd, c.off_host, far, g);
+    return g.ext;
+  };
+  auto pick = [&](bool ghost, uint32_t far) {
+    const uint32_t ext = segments(far);
+    const size_t bytes = tab + (static_cast<size_t>(ext) + rows) * sizeof(T);
+    if (bytes > kOcLds) return false;
+    void (*k)(OcArgs<T>) = nullptr;
+    if (c.jacobi)
+      k = c.wide ? oc_kernel<T, true, kVecW<T> >(ghost, cpv, tpc, ext - rows, c.dia.code != nullptr) : nullptr;
+    else
+      k = c.wide ? oc_kernel<T, false, kVecW<T> >(ghost, cpv, tpc, ext - rows, c.dia.code != nullptr) : nullptr;
+    if (!k) return false;
+    pl.kernel = k;
+    pl.ghost = ghost;
+    pl.far = far;
+    pl.ext = ext;
+    pl.lds = bytes;
+    return true;
+  };
+  if (pick(true, 0)) return true;
+  uint32_t far = 0, nfar = 0;
+  for (uint32_t i = 0; i < nd; ++i)
+    if (static_cast<uint32_t>(std::abs(c.off_host[i])) >= rows) {
+      far |= 1u << i;
+      ++nfar;
+    }
+  const uint32_t least = wg_tiles(false) * kBlock;
+  if (nfar > 2 || least == 0) return false;
+  pl.reach = (static_cast<uint32_t>(reach_rows) + least - 1) / least + 1;
+  if (2 * pl.reach + 1 > 2 * kWave) return false;
+  return pick(false, far);
+}
+
+}  // namespace
+
+template <typename T>
+int onchip_cg(const OnchipCg<T>& c, Workspace& ws, hipStream_t s, KState* fin, Onchip* outcome)
+{
+  *outcome = Onchip::kNo;
+  t_on_chip = 0;
+  OcPlan<T> pl;
+  if (!oc_plan(c, pl)) return VCLHIP_SUCCESS;
+  int dev = 0;
+  VCLHIP_HIP(hipGetDevice(&dev));
+  if (dev < 0 || dev >= 64) return VCLHIP_SUCCESS;
+  std::unique_lock<std::mutex> slot(g_slot[dev], std::try_to_lock);
+  if (!slot.owns_lock()) return VCLHIP_SUCCESS;
+  VCLHIP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(pl.kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                 static_cast<int>(pl.lds)));
+  int per_cu = 0;
+  VCLHIP_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(pl.kernel), kOcThreads,
+                                                          pl.lds));
+  if (per_cu < 1) return VCLHIP_SUCCESS;
+  // the exchange lines, the flags and the abort word, cleared before the launch
+  struct Shared {
+    unsigned long long lines[2 * kOwners * kOcLine];
+    uint32_t flags[kOwners * 16];
+    uint32_t abort;
+  };
+  Shared* sh;
+  T* ap2 = nullptr;
+  if (!ws.try_alloc(&sh, 1) || (pl.ghost && !ws.try_alloc(&ap2, c.n))) return VCLHIP_SUCCESS;
+  VCLHIP_TRY(vclhip_fill_zero(sh, sizeof(Shared), s));
+  OcArgs<T> a{};
+  a.n = c.n;
+  a.nd = c.dia.nd;
+  a.gp = cg_prod_chunks(c.n);
+  a.m = pl.m;
+  a.nwg = pl.nwg;
+  a.far = pl.far;
+  a.ext = pl.ext;
+  a.reach = pl.reach;
+  for (uint32_t i = 0; i < c.dia.nd; ++i) a.off[i] = c.off_host[i];
+  a.val = c.dia.val;
+  a.code = c.dia.code;
+  a.table = c.dia.table;
+  a.x = c.x;
+  a.r = c.r;
+  a.p = c.p;
+  a.d = c.d;
+  a.ex0 = pl.ghost ? ap2 : const_cast<T*>(c.p);
+  a.ex1 = c.Ap;
+  a.st = c.st;
+  a.lines = sh->lines;
+  a.flags = sh->flags;
+  a.abort = &sh->abort;
+  a.wait = wait_ticks();
+  hipLaunchKernelGGL(pl.kernel, dim3(pl.nwg), dim3(kOcThreads), pl.lds, s, a);
+  VCLHIP_TRY(check_launch("onchip_cg_kernel"));
+  uint32_t aborted = 0;
+  VCLHIP_HIP(hipMemcpyAsync(&aborted, &sh->abort, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+  VCLHIP_HIP(hipMemcpyAsync(fin, c.st, sizeof(KState), hipMemcpyDeviceToHost, s));
+  VCLHIP_HIP(hipStreamSynchronize(s));
+  *outcome = aborted ? Onchip::kAborted : Onchip::kDone;
+  t_on_chip = aborted ? 2 : 1;
+  return VCLHIP_SUCCESS;
+}
+
+template int onchip_cg<double>(const OnchipCg<double>&, Workspace&, hipStream_t, KState*, Onchip*);
+template int onchip_cg<float>(const OnchipCg<float>&, Workspace&, hipStream_t, KState*, Onchip*);
+
+}  // namespace vclhip
+
+extern "C" {
+
+int vclhip_onchip_wait_limit(double microseconds)
+{
+  vclhip::t_wait_us = microseconds;
+  return VCLHIP_SUCCESS;
+}
+
+int vclhip_onchip_last(void)
+{
+  const int v = vclhip::t_on_chip;
+  vclhip::t_on_chip = 0;
+  return v;
+}
+
+}  // extern "C"
