@@ -440,9 +440,11 @@ typedef struct vclhip_solver_params {
                                         BiCGStab without a preconditioner: 0 = automatic (a small
                                         system runs four kernels per iteration), 1 = six; the
                                         results are the same bit for bit.
-                                        CG: 0 = automatic (a small system on a DIA operator runs one
-                                        kernel per iteration), 1 = at least two kernels per
-                                        iteration; the results are the same bit for bit */
+                                        CG: 0 = automatic (a system on a DIA operator whose vectors fit
+                                        the compute units' registers runs all iterations in one
+                                        kernel, a small one otherwise one kernel per iteration),
+                                        1 = at least two kernels per iteration; the results are the
+                                        same bit for bit */
   double* history_host;              /* optional: per-iteration convergence quantity (may be NULL) */
   uint32_t history_len;
   /* optional monitor, called once per iteration with the device solution and the relative residual
@@ -505,7 +507,8 @@ typedef struct vclhip_solver_result {
                          VCLHIP_INNER_SELL64, VCLHIP_INNER_SELL64_D16, VCLHIP_INNER_DIA or
                          VCLHIP_INNER_DIA_CODED */
   uint32_t kernels_per_iter;  /* CG: kernels launched per iteration after the first (1 in fused mode,
-                                 2 in compact mode, else 3); BiCGStab: 4 in compact mode, 6 pipelined,
+                                 2 in compact mode, else 3; a solve that runs all iterations in one
+                                 kernel reports the mode it would take otherwise); BiCGStab: 4 in compact mode, 6 pipelined,
                                  8 with the reference's Jacobi recurrences; 0 from the other solvers */
 } vclhip_solver_result;
 #define VCLHIP_USED_AS_GIVEN 0

@@ -1,0 +1,125 @@
+"""CG with all iterations in one launch (onchip_cg.hip) against the kernel-per-step modes, bit for bit."""
+import ctypes
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+NOT_RUN, RAN, GAVE_UP = 0, 1, 2
+
+
+def band(n, offsets, values, seed=0):
+    """Symmetric diagonally dominant band matrix in CSR: offsets > 0 given, `values` distinct numbers
+    on every diagonal (0: all different)."""
+    import scipy.sparse as sp
+    rng = np.random.default_rng(seed)
+    M = sp.csr_matrix((n, n))
+    for o in offsets:
+        if o < n:
+            v = -rng.uniform(0.5, 1.0, n - o) if values == 0 else -1.0 / (1.0 + np.arange(n - o) % values)
+            D = sp.diags(v, o, shape=(n, n))
+            M = M + D + D.T
+    top = float(np.asarray(abs(M).sum(axis=1)).max()) if M.nnz else 1.0
+    d = top + 0.05 + (rng.uniform(0, 1, n) if values == 0 else (np.arange(n) % values) * 0.5)
+    M = sp.csr_matrix(M + sp.diags(d))
+    M.sort_indices()
+    return M.indptr.astype(np.uint32), M.indices.astype(np.uint32), M.data.astype(np.float64)
+
+
+def run(vh, A, b, dtype, **kw):
+    db, dx = vh.DeviceArray.from_numpy(b.astype(dtype)), vh.DeviceArray.zeros(b.size, dtype)
+    hist = np.zeros(kw["max_iters"])
+    vh.lib().vclhip_onchip_last()
+    res = vh.cg(A, db, dx, history=hist, **kw)
+    return dx.to_numpy(), res, hist, vh.lib().vclhip_onchip_last()
+
+
+def check(vh, A, b, dtype, want, **kw):
+    x0, r0, h0, mode = run(vh, A, b, dtype, **kw)
+    x1, r1, h1, other = run(vh, A, b, dtype, variant=1, **kw)
+    assert mode == want and other == NOT_RUN
+    assert r0.iters == r1.iters and np.array_equal(r0.error, r1.error, equal_nan=True) and r0.converged == r1.converged
+    assert r0.kernels_per_iter in (1, r1.kernels_per_iter)
+    assert np.array_equal(x0, x1, equal_nan=True) and np.array_equal(h0, h1, equal_nan=True)
+    return r0
+
+
+# rows: the edges of tiles, of one owner per chunk (65536), of the workgroup's share (131072), of the
+# chunk length (524288) and of the value dictionary (262144); offsets: inside a workgroup's rows, just
+# around them, and far (read from memory from two rows per lane on).
+CASES = {
+    "one_row": (1, [], 1, True), "tile_edge_255": (255, [1], 1, True), "tile_edge_257": (257, [1, 16], 0, True),
+    "owners_65535": (65535, [1, 255], 0, True), "owners_65536": (65536, [1, 256], 0, True),
+    "owners_65537": (65537, [1, 256], 0, True), "two_tiles_131073": (131073, [1, 300, 6000], 0, True),
+    "coded_262144": (262144, [1, 64, 4096], 1, True), "two_values_262145": (262145, [1, 64, 4096], 2, True),
+    "regs_300001": (300001, [1, 547], 0, True), "halo_524289": (524289, [1, 80, 6400], 0, True),
+    "halo_one_value": (700001, [1, 88, 7744], 1, True), "halo_codes": (700003, [1, 88, 7744], 3, True),
+    "halo_wide": (1048577, [1, 101, 10201], 0, True), "halo_wide_one_value": (1500001, [1, 114, 13000], 1, True),
+    "far_middle": (700001, [1, 7000, 7744], 1, False), "eight_diagonals": (70001, [1, 3, 40, 900], 0, False),
+}
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("precond", [0, 1])
+@pytest.mark.parametrize("case", list(CASES))
+def test_equals_the_kernel_per_step_modes(dev, vh, case, precond, dtype):
+    """x, iterations, error and history of the one-launch solve equal those of the launched modes bit
+    for bit: every partial sum is formed in the same order.  Systems it does not take run launched."""
+    n, offsets, values, fits = CASES[case]
+    rp, col, val = band(n, offsets, values, seed=n)
+    A = vh.CsrMatrix(rp, col, val, dtype=dtype)
+    tol = 1e-9 if dtype == np.float64 else 1e-4
+    r = check(vh, A, vh.random_uniform(4, n), dtype, RAN if fits else NOT_RUN, precond=precond, tol=tol, max_iters=400)
+    assert r.converged
+
+
+def test_nonsymmetric_reach(dev, vh):
+    """Diagonals on one side only (an upper band; CG does not converge on it): the same iterates up to
+    the limit."""
+    import scipy.sparse as sp
+    n = 600001
+    M = sp.csr_matrix(sp.diags([np.full(n, 4.0), -np.ones(n - 1), -np.ones(n - 7000)], [0, 1, 7000]))
+    A = vh.CsrMatrix(M.indptr.astype(np.uint32), M.indices.astype(np.uint32), M.data)
+    check(vh, A, vh.random_uniform(6, n), np.float64, RAN, tol=1e-30, max_iters=37)
+
+
+def test_more_iterations_than_one_launch_runs(dev, vh):
+    """A launch ends after 4096 iterations and the next one goes on: 1-D and 2-D systems (exchanged rows
+    of the operator's product, and of the direction) beyond that, and ends at 4096 exactly."""
+    for n, offsets in ((9001, [1]), (525001, [1, 6000])):
+        rp, col, val = band(n, offsets, 1)
+        rows = np.repeat(np.arange(n), np.diff(rp.astype(np.int64)))
+        val[col.astype(np.int64) == rows] -= 0.05 - 1e-9  # nearly singular: thousands of iterations
+        A = vh.CsrMatrix(rp, col, val)
+        for limit in (4095, 4096, 4097, 4610):
+            r = check(vh, A, vh.random_uniform(8, n), np.float64, RAN, tol=0.0, max_iters=limit)
+            assert r.iters == limit
+
+
+def test_values_that_are_not_finite(dev, vh):
+    """NaN and infinity in the right-hand side spread as in the launched modes."""
+    rp, col, val = band(140001, [1, 375], 0)
+    A = vh.CsrMatrix(rp, col, val)
+    for bad in (np.nan, np.inf):
+        b = vh.random_uniform(2, 140001)
+        b[70000] = bad
+        for pc in (0, 1):
+            check(vh, A, b, np.float64, RAN, precond=pc, tol=1e-9, max_iters=9)
+
+
+def test_gives_up_when_its_workgroups_do_not_meet(dev, vh):
+    """With a wait limit of zero every first unsuccessful look gives up: the launched modes take over
+    from the start, with their results."""
+    limit = vh.lib().vclhip_onchip_wait_limit
+    limit.argtypes = [ctypes.c_double]
+    for n, offsets in ((65536, [1, 256]), (700001, [1, 88, 7744])):
+        rp, col, val = band(n, offsets, 1)
+        A = vh.CsrMatrix(rp, col, val)
+        b = vh.random_uniform(3, n)
+        limit(0.0)
+        try:
+            check(vh, A, b, np.float64, GAVE_UP, tol=1e-9, max_iters=400)
+        finally:
+            limit(-1.0)
+        check(vh, A, b, np.float64, RAN, tol=1e-9, max_iters=400)

@@ -232,19 +232,6 @@ __device__ __forceinline__ void block_sum_partials_k(const A* const (&p)[K], con
   block_combine_k<K, A>(s, out);
 }
 
-template <typename A>
-__device__ __forceinline__ void block_sum_partials3(const A* pa, uint32_t na, const A* pb, uint32_t nb,
-                                                    const A* pc, uint32_t nc, A& ra, A& rb, A& rc)
-{
-  const A* const p[3] = {pa, pb, pc};
-  const uint32_t count[3] = {na, nb, nc};
-  A out[3];
-  block_sum_partials_k<3, A>(p, count, out);
-  ra = out[0];
-  rb = out[1];
-  rc = out[2];
-}
-
 // [begin, end) of the lw-th of G chunks of n elements with both ends on multiples of W (the last
 // chunk also takes the tail), so that W-wide vector accesses of a W*sizeof(T)-aligned array stay
 // aligned.

@@ -147,11 +147,11 @@ __device__ __forceinline__ bool dia_set_insert(unsigned long long* slots, unsign
 
 // Pass 1: workgroup (g, d) collects the distinct values of diagonal d over rows g*kBlock + tid,
 // stepping by gridDim.x*kBlock, into sets[(d * gridDim.x + g) * kDiaDictSlots ...]; more than
-// kDiaDictSlots of them raise *overflow.
+// kDiaDictSlots of them make *distinct larger than that.
 template <typename T>
 __global__ __launch_bounds__(kBlock) void dia_dict_collect_kernel(const T* __restrict__ val, uint32_t n,
                                                                   unsigned long long* __restrict__ sets,
-                                                                  uint32_t* __restrict__ overflow)
+                                                                  uint32_t* __restrict__ distinct)
 {
   __shared__ unsigned long long slots[kDiaDictSlots];
   __shared__ uint32_t full;
@@ -172,16 +172,17 @@ __global__ __launch_bounds__(kBlock) void dia_dict_collect_kernel(const T* __res
     if (stop_now) break;
   }
   if (tid < kDiaDictSlots) sets[(static_cast<size_t>(d) * gridDim.x + blockIdx.x) * kDiaDictSlots + tid] = slots[tid];
-  if (tid == 0 && full) *overflow = 1u;
+  if (tid == 0 && full) *distinct = kDiaDictSlots + 1;
 }
 
 // Pass 2: workgroup d merges the groups' sets of diagonal d into its table (entry 0 the zero of an
-// absent entry, unused entries zero) and keeps the keys for pass 3.
+// absent entry, unused entries zero) and keeps the keys for pass 3; *distinct becomes the largest
+// number of values in a table.
 template <typename T>
 __global__ __launch_bounds__(kBlock) void dia_dict_merge_kernel(const unsigned long long* __restrict__ sets,
                                                                 uint32_t groups, T* __restrict__ table,
                                                                 unsigned long long* __restrict__ keys,
-                                                                uint32_t* __restrict__ overflow)
+                                                                uint32_t* __restrict__ distinct)
 {
   __shared__ unsigned long long slots[kDiaDictSlots];
   __shared__ uint32_t full;
@@ -200,7 +201,8 @@ __global__ __launch_bounds__(kBlock) void dia_dict_merge_kernel(const unsigned l
     table[d * kDiaCodes + tid] = dia_value<T>(k);
     keys[d * kDiaCodes + tid] = k;
   }
-  if (tid == 0 && full) *overflow = 1u;
+  if (tid < kDiaDictSlots && slots[tid] != 0ull) atomicMax(distinct, tid + 1);
+  if (tid == 0 && full) atomicMax(distinct, kDiaDictSlots + 1);
 }
 
 // Pass 3: code[d * n + row] = the index of the row's value in its diagonal's table.
@@ -254,15 +256,16 @@ static int build_dia_codes(DiaDev<T>& dia, void* extra, Workspace& ws, uint32_t*
   VCLHIP_TRY(check_launch("dia_dict_collect_kernel"));
   hipLaunchKernelGGL(dia_dict_merge_kernel<T>, dim3(nd), dim3(kBlock), 0, s, sets, groups, table, keys, flag);
   VCLHIP_TRY(check_launch("dia_dict_merge_kernel"));
-  uint32_t hover = 0;
-  VCLHIP_HIP(hipMemcpyAsync(&hover, flag, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+  uint32_t distinct = 0;
+  VCLHIP_HIP(hipMemcpyAsync(&distinct, flag, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
   VCLHIP_HIP(hipStreamSynchronize(s));
-  if (hover) return VCLHIP_SUCCESS;
+  if (distinct > kDiaDictSlots) return VCLHIP_SUCCESS;
   hipLaunchKernelGGL(dia_encode_kernel<T>, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, dia.val, n, nd, keys,
                      code);
   VCLHIP_TRY(check_launch("dia_encode_kernel"));
   dia.code = code;
   dia.table = table;
+  dia.distinct = distinct;
   *coded = true;
   return VCLHIP_SUCCESS;
 }
@@ -337,6 +340,7 @@ static int build_dia(const vclhip_csr* A, Workspace& ws, hipStream_t s, double m
   if (hover) return VCLHIP_SUCCESS;
   out->val = val;
   out->off = arr.off;
+  for (uint32_t i = 0; i < nd && i < kDiaGroup; ++i) out->first_off[i] = offs[i];
   out->n_rows = n;
   out->nd = nd;
   out->code = nullptr;

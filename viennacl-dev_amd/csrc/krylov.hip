@@ -14,7 +14,10 @@
 #include <mutex>
 #include <vector>
 
+#include "cg_sums.hpp"
 #include "internal.hpp"
+#include "krylov_state.hpp"
+#include "onchip_cg.hpp"
 #include "solver.hpp"
 #include "spmv_kernels.hpp"
 #include "dia.hpp"
@@ -23,18 +26,6 @@ namespace vclhip {
 
 // ------------------------------------------------------------------ solver state
 
-enum : uint32_t {
-  kFlagDone = 1u,       // every kernel of the solve returns at once
-  kFlagFinishing = 2u,  // BiCGStab: the final vector update is pending, everything else stops
-  // Mixed-precision CG.  An iteration that asks for an FP64 correction sets Pause (the remaining
-  // iterations of the chunk return at once) and clears NoPause (the correction kernels at the end of
-  // the chunk run).  The correction clears TailIdle while it refreshes the FP32 state.
-  kFlagPause = 4u,
-  kFlagNoPause = 8u,
-  kFlagTailIdle = 16u,
-};
-
-constexpr uint32_t kSlots = 8;  // partial-sum slots of kMaxPartials doubles each
 // Compact CG: at most this many partials read by all update workgroups together per iteration
 // (1 Mi: the 512^2 diffusion operator, 256 update workgroups reading 2304 partials each, runs 9%
 // faster than with three kernels; at n = 1 M the reads would cost more than the kernel saved).
@@ -45,41 +36,6 @@ constexpr uint64_t kCompactPartialReads = 1ull << 20;
 // 11.0 against 12.0 at 518 K (350^2), even at 555-832 K (50^3, 392^2), 17.6 against 14.6 at 1.4 M
 // (450^2).
 constexpr uint64_t kFusedPartialReads = 1ull << 19;
-
-struct KState {
-  double alpha, beta, omega;
-  double rr;        // CG: <r,r> or <r,M^-1 r>;  BiCGStab: <r,r0*>
-  double nrs;       // CG: norm of the right-hand side squared;  BiCGStab: ||b||
-  double res;       // BiCGStab residual-norm estimate
-  double ap_r0;     // BiCGStab <Ap,r0*> of the current iteration
-  double tol, abs_tol;
-  double* history;  // device array or null
-  uint32_t history_len;
-  uint32_t iter, max_iters;
-  uint32_t flags;
-  uint32_t converged;
-  uint32_t final_mode;        // BiCGStab: 0 full update, 1 converged (x only), 2 last iteration (full)
-  uint32_t rr_from_partials;  // BiCGStab: <r,r0*> comes from the previous vector update's partials
-  uint32_t breakdown;
-  // mixed-precision CG
-  double rr2;       // FP32 recursive <r,r>
-  double rr_ref;    // <r,r> after the last FP64 correction (reliable update)
-  float inner, initial;  // reference schedule: FP32 <r,r> and its value at the last restart
-  float inner_tol;
-  uint32_t updates;      // FP64 corrections done
-  uint32_t iter2[2];     // CG, compact mode: iteration count, read from [k & 1] and written to the other
-};
-
-__host__ __device__ __forceinline__ double* slot_ptr(double* part, uint32_t slot) { return part + slot * kMaxPartials; }
-__host__ __device__ __forceinline__ const double* slot_ptr(const double* part, uint32_t slot)
-{
-  return part + slot * kMaxPartials;
-}
-
-__device__ __forceinline__ void record_history(KState* st, uint32_t iter, double v)
-{
-  if (st->history && iter >= 1 && iter <= st->history_len) st->history[iter - 1] = v;
-}
 
 // ------------------------------------------------------------------ epilogues
 
@@ -157,7 +113,7 @@ __global__ __launch_bounds__(kBlock) void cg_init_kernel(uint32_t n, const T* __
 {
   const uint32_t lw = xcd_logical_block();
   uint32_t c0, c1;
-  chunk_range_w(n, W, lw, gridDim.x, c0, c1);
+  cg_vec_rows(n, lw, c0, c1);
   double acc[1] = {0};
   for_packs<W>(c0, c1, [&](uint32_t i, auto w) {
     constexpr int V = decltype(w)::value;
@@ -186,7 +142,7 @@ __global__ __launch_bounds__(kBlock) void cg_setup_kernel(KState* __restrict__ s
                                                           uint32_t g_vec, uint32_t g_prod)
 {
   double bb, ApAp, pAp;
-  block_sum_partials3(slot_ptr(part, 0), g_vec, slot_ptr(part, 1), g_prod, slot_ptr(part, 2), g_prod, bb, ApAp, pAp);
+  owner_sums3(slot_ptr(part, 0), g_vec, slot_ptr(part, 1), g_prod, slot_ptr(part, 2), g_prod, bb, ApAp, pAp);
   if (threadIdx.x != 0) return;
   double nrs;
   if (Jac) {
@@ -229,7 +185,7 @@ __global__ __launch_bounds__(kBlock) void cg_update_kernel(uint32_t n, T* __rest
   const T beta = static_cast<T>(st->beta);
   const uint32_t lw = xcd_logical_block();
   uint32_t c0, c1;
-  chunk_range_w(n, W, lw, gridDim.x, c0, c1);
+  cg_vec_rows(n, lw, c0, c1);
   double acc[1] = {0};
   for_packs<W>(c0, c1, [&](uint32_t i, auto w) {
     constexpr int V = decltype(w)::value;
@@ -261,7 +217,7 @@ __global__ __launch_bounds__(kBlock) void cg_iter_kernel(KState* __restrict__ st
 {
   if (st->flags & kFlagDone) return;
   double rr, ApAp, pAp;
-  block_sum_partials3(slot_ptr(part, 0), g_vec, slot_ptr(part, 1), g_prod, slot_ptr(part, 2), g_prod, rr, ApAp, pAp);
+  owner_sums3(slot_ptr(part, 0), g_vec, slot_ptr(part, 1), g_prod, slot_ptr(part, 2), g_prod, rr, ApAp, pAp);
   if (threadIdx.x != 0) return;
   const uint32_t iter = st->iter + 1;
   st->iter = iter;
@@ -296,7 +252,7 @@ __global__ __launch_bounds__(kBlock) void cg_step_kernel(uint32_t n, T* __restri
 {
   if (st->flags & kFlagDone) return;
   double rr, ApAp, pAp;
-  block_sum_partials3(slot_ptr(part, par ? 3u : 0u), g_vec, slot_ptr(part, 1), g_prod, slot_ptr(part, 2), g_prod,
+  owner_sums3(slot_ptr(part, par ? 3u : 0u), g_vec, slot_ptr(part, 1), g_prod, slot_ptr(part, 2), g_prod,
                       rr, ApAp, pAp);
   const uint32_t iter = st->iter2[par] + 1;
   const bool conv = fabs(rr / st->nrs) < st->tol * st->tol || fabs(rr) < st->abs_tol * st->abs_tol;
@@ -321,7 +277,7 @@ __global__ __launch_bounds__(kBlock) void cg_step_kernel(uint32_t n, T* __restri
   const T tb = static_cast<T>(beta);
   const uint32_t lw = xcd_logical_block();
   uint32_t c0, c1;
-  chunk_range_w(n, W, lw, gridDim.x, c0, c1);
+  cg_vec_rows(n, lw, c0, c1);
   double acc[1] = {0};
   for_packs<W>(c0, c1, [&](uint32_t i, auto w) {
     constexpr int V = decltype(w)::value;
@@ -382,23 +338,26 @@ __global__ __launch_bounds__(kBlock) void cg_fused_kernel(uint32_t n, T* __restr
   const uint32_t tid = threadIdx.x;
   const uint32_t lw = xcd_logical_block();
 
-  // ---- loads issued ahead of the scalar step: first the partial sums it reduces (up to
-  // kFusedPartials per slot and lane; lane t takes entries t, t + 256, ... as block_sum_partials_k)
+  // ---- loads issued ahead of the scalar step: first the partial sums it reduces (lane o takes those
+  // of owner o as owner_sums_k, the first kFusedPartials of each slot here)
   const double* const ps[3] = {slot_ptr(part, par ? 3u : 0u), slot_ptr(part, par ? 4u : 1u),
                                slot_ptr(part, par ? 5u : 2u)};
   const uint32_t pc[3] = {g_vec, g_prod, g_prod};
+  uint32_t pb[3], pe[3];
+#pragma unroll
+  for (int q = 0; q < 3; ++q) owner_range(pc[q], tid, pb[q], pe[q]);
   double pv[kFusedPartials][3];
 #pragma unroll
   for (uint32_t b = 0; b < kFusedPartials; ++b)
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
       // unconditional (clamped) loads, so that no sum is placed next to its load and waits for it
-      const uint32_t i = tid + b * kBlock;
+      const uint32_t i = pb[q] + b;
       pv[b][q] = ps[q][i < pc[q] ? i : pc[q] - 1];
     }
   const bool has_vec = lw < g_vec;
   uint32_t c0 = 0, c1 = 0;
-  if (has_vec) chunk_range_w(n, W, lw, g_vec, c0, c1);
+  if (has_vec) cg_vec_rows(n, lw, c0, c1);
   const uint32_t packed_end = c0 + ((c1 - c0) / W) * W;
   Pack<W, T> fp[kFusedPacks], fr[kFusedPacks], fx[kFusedPacks], fa[kFusedPacks], fd[kFusedPacks];
 #pragma unroll
@@ -445,19 +404,17 @@ __global__ __launch_bounds__(kBlock) void cg_fused_kernel(uint32_t n, T* __restr
 
   if (flags & kFlagDone) return;  // the same value for every lane: all return or none
 
-  // ---- the scalar step of iteration k: the partial sums added in block_sum_partials_k's order
+  // ---- the scalar step of iteration k: the partial sums added in owner_sums_k's order
   double sums[3] = {0, 0, 0}, red3[3];
 #pragma unroll
   for (uint32_t b = 0; b < kFusedPartials; ++b)
 #pragma unroll
     for (int q = 0; q < 3; ++q)
-      if (tid + b * kBlock < pc[q]) sums[q] += pv[b][q];
-  const uint32_t pmax = g_vec > g_prod ? g_vec : g_prod;
-  for (uint32_t i = tid + kFusedPartials * kBlock; i < pmax; i += kBlock)
+      if (pb[q] + b < pe[q]) sums[q] += pv[b][q];
 #pragma unroll
-    for (int q = 0; q < 3; ++q)
-      if (i < pc[q]) sums[q] += ps[q][i];
-  block_combine_k<3, double>(sums, red3);
+  for (int q = 0; q < 3; ++q)
+    for (uint32_t i = pb[q] + kFusedPartials; i < pe[q]; ++i) sums[q] += ps[q][i];
+  owner_tree_k<3, double>(sums, red3);
   const double rr = red3[0], ApAp = red3[1], pAp = red3[2];
   const uint32_t iter = iter_prev + 1;
   const bool conv = fabs(rr / nrs) < tol * tol || fabs(rr) < abs_tol * abs_tol;
@@ -1390,30 +1347,32 @@ static int cg_solve(const M* Ain, const T* b, T* x, int precond, const vclhip_so
   }
   int used_dia = 0;
   VCLHIP_TRY(dia_operator(op, ws, s, P, &used_dia));
-  KState h;
-  init_state(h, P, hist);
-  VCLHIP_TRY(upload_state(st, h, s));
-
-  const uint32_t gv = solver_vec_grid(n);
+  const uint32_t gv = cg_vec_chunks(n);
   const bool v2 = aligned16({b, x});  // workspace vectors are 256-byte aligned
   // setup: x = 0, r = b, p = M^-1 b, Ap = A p, scalars
-  if (jac)
-    VCLHIP_LAUNCH_W(v2, (cg_init_kernel<T, true, kVecW<T> >), (cg_init_kernel<T, true, 1>), gv, s, n, b, x, r, p,
-                    d, part);
-  else
-    VCLHIP_LAUNCH_W(v2, (cg_init_kernel<T, false, kVecW<T> >), (cg_init_kernel<T, false, 1>), gv, s, n, b, x, r, p,
-                    d, part);
-  VCLHIP_TRY(check_launch("cg_init_kernel"));
-  if (jac)
-    op.launch(s, p, EpiCg<T, true>{Ap, p, d}, slot_ptr(part, 1), nullptr, 0u);
-  else
-    op.launch(s, p, EpiCg<T, false>{Ap, p, d}, slot_ptr(part, 1), nullptr, 0u);
-  VCLHIP_TRY(check_launch("cg prod"));
-  if (jac)
-    hipLaunchKernelGGL(cg_setup_kernel<true>, dim3(1), dim3(kBlock), 0, s, st, part, gv, op.grid);
-  else
-    hipLaunchKernelGGL(cg_setup_kernel<false>, dim3(1), dim3(kBlock), 0, s, st, part, gv, op.grid);
-  VCLHIP_TRY(check_launch("cg_setup_kernel"));
+  auto start = [&]() -> int {
+    KState h;
+    init_state(h, P, hist);
+    VCLHIP_TRY(upload_state(st, h, s));
+    if (jac)
+      VCLHIP_LAUNCH_W(v2, (cg_init_kernel<T, true, kVecW<T> >), (cg_init_kernel<T, true, 1>), gv, s, n, b, x, r, p,
+                      d, part);
+    else
+      VCLHIP_LAUNCH_W(v2, (cg_init_kernel<T, false, kVecW<T> >), (cg_init_kernel<T, false, 1>), gv, s, n, b, x, r, p,
+                      d, part);
+    VCLHIP_TRY(check_launch("cg_init_kernel"));
+    if (jac)
+      op.launch(s, p, EpiCg<T, true>{Ap, p, d}, slot_ptr(part, 1), nullptr, 0u);
+    else
+      op.launch(s, p, EpiCg<T, false>{Ap, p, d}, slot_ptr(part, 1), nullptr, 0u);
+    VCLHIP_TRY(check_launch("cg prod"));
+    if (jac)
+      hipLaunchKernelGGL(cg_setup_kernel<true>, dim3(1), dim3(kBlock), 0, s, st, part, gv, op.grid);
+    else
+      hipLaunchKernelGGL(cg_setup_kernel<false>, dim3(1), dim3(kBlock), 0, s, st, part, gv, op.grid);
+    return check_launch("cg_setup_kernel");
+  };
+  VCLHIP_TRY(start());
 
   uint32_t* flags = &st->flags;
   auto launch_update = [&]() {
@@ -1483,7 +1442,17 @@ static int cg_solve(const M* Ain, const T* b, T* x, int precond, const vclhip_so
   };
   KState fin;
   const bool no_alloc = arena != nullptr;
-  if (compact) {
+  // On-chip mode: all iterations in one launch where the vectors fit the CUs' registers and LDS, with
+  // the same results.  Not where the caller asks for a form of launches (graph, variant 1) or watches
+  // the iterations.
+  Onchip on_chip = Onchip::kNo;
+  if (op.fmt == OpFormat::Dia && op.grid == cg_prod_chunks(n) && P->variant == 0 && !P->use_graph && !P->monitor) {
+    VCLHIP_TRY(onchip_cg<T>({n, op.dia, jac, v2, x, r, p, Ap, d, st}, ws, s, &fin, &on_chip));
+    if (on_chip == Onchip::kAborted) VCLHIP_TRY(start());
+  }
+  if (on_chip == Onchip::kDone) {
+    // x and fin are there
+  } else if (compact) {
     launch_update();  // the update of iteration 0; iteration k then closes with that of k + 1
     VCLHIP_TRY(check_launch("cg update"));
     if (fused) {

@@ -1,0 +1,35 @@
+// onchip_cg.hpp -- CG on a DIA operator in one launch: every vector of the solve lives in the
+// registers and LDS of the CUs and only boundary rows and inner products travel between them.
+#pragma once
+
+#include "krylov_state.hpp"
+#include "solver.hpp"
+
+namespace vclhip {
+
+// What a solve that stands right after cg_setup_kernel hands over: x = 0, r, p and A p of the first
+// direction in memory, the scalars in *st.
+template <typename T>
+struct OnchipCg {
+  uint32_t n;
+  DiaDev<T> dia;
+  bool jacobi;
+  bool wide;  // the vector kernels' 16-byte packs (their partial sums' grouping)
+  T* x;
+  T* r;
+  T* p;
+  T* Ap;
+  const T* d;
+  KState* st;
+};
+
+enum class Onchip { kNo, kDone, kAborted };
+
+// Runs the iterations to the end if the system fits.  kNo: it does not (or another solve of this
+// process holds the device's on-chip slot): nothing was launched and the solve stands as before.
+// kAborted: the workgroups could not all run at once within the wait limit; the vectors and *st are
+// then undefined and the caller starts over with the other modes.  kDone: x is written and *fin is the final state.
+template <typename T>
+int onchip_cg(const OnchipCg<T>& c, Workspace& ws, hipStream_t s, KState* fin, Onchip* outcome);
+
+}  // namespace vclhip

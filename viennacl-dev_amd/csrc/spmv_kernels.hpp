@@ -339,6 +339,8 @@ struct DiaDev {
   uint32_t nd;
   const uint8_t* __restrict__ code = nullptr;
   const T* __restrict__ table = nullptr;
+  uint32_t distinct = 0;              // values in the longest table, without the absent entry's zero
+  int32_t first_off[kDiaGroup] = {};  // the first nd of the offsets, for the host and as kernel arguments
 };
 
 // One lane per row over the diagonals in offset order, i.e. the row's entries in column order, zero
