@@ -123,3 +123,29 @@ def test_gives_up_when_its_workgroups_do_not_meet(dev, vh):
         finally:
             limit(-1.0)
         check(vh, A, b, np.float64, RAN, tol=1e-9, max_iters=400)
+
+
+@pytest.mark.parametrize("case", ["diffusion_small", "diffusion_halo", "laplace_one_value", "sixteen_rows_a_lane", "limit"])
+def test_mixed_inner_iterations(dev, vh, case):
+    """The mixed solver's FP32 inner iterations between two FP64 corrections in one launch: x, counts,
+    error and history equal those of the launched ones bit for bit."""
+    k = lambda n, s: np.exp(s * vh.random_normal(3, n))
+    rp, col, val = {"diffusion_small": lambda: vh.diffusion(31, 29, 23, k(31 * 29 * 23, 1.0)),
+                    "diffusion_halo": lambda: vh.diffusion(95, 91, 89, k(95 * 91 * 89, 1.0)),
+                    "laplace_one_value": lambda: vh.laplace_3d(120, 118, 110),
+                    "sixteen_rows_a_lane": lambda: vh.diffusion(161, 159, 150, k(161 * 159 * 150, 0.3)),
+                    "limit": lambda: vh.fdm_laplace_2d(300, 301)}[case]()
+    n = rp.size - 1
+    A, b = vh.CsrMatrix(rp, col, val), vh.random_uniform(5, n)
+    kw = dict(tol=1e-10, max_iters=150 if case == "limit" else 4000, mixed_mode=1)
+    out = []
+    for variant in (0, 1):
+        db, dx, hist = vh.DeviceArray.from_numpy(b), vh.DeviceArray.zeros(n, np.float64), np.zeros(kw["max_iters"])
+        vh.lib().vclhip_onchip_last()
+        res = vh.mixed_cg(A, db, dx, variant=variant, history=hist, **kw)
+        out.append((dx.to_numpy(), hist, res, vh.lib().vclhip_onchip_last()))
+    (x0, h0, r0, m0), (x1, h1, r1, m1) = out
+    assert (m0, m1) == (RAN, NOT_RUN)
+    assert r0.iters == r1.iters and r0.restarts == r1.restarts and r0.error == r1.error and r0.converged == r1.converged
+    assert np.array_equal(x0, x1) and np.array_equal(h0, h1)
+    assert r0.converged == (case != "limit") and r0.restarts >= 1

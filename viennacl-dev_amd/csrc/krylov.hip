@@ -1447,7 +1447,7 @@ static int cg_solve(const M* Ain, const T* b, T* x, int precond, const vclhip_so
   // the iterations.
   Onchip on_chip = Onchip::kNo;
   if (op.fmt == OpFormat::Dia && op.grid == cg_prod_chunks(n) && P->variant == 0 && !P->use_graph && !P->monitor) {
-    VCLHIP_TRY(onchip_cg<T>({n, op.dia, jac, v2, x, r, p, Ap, d, st}, ws, s, &fin, &on_chip));
+    VCLHIP_TRY(onchip_cg<T>({n, op.dia, jac, v2, x, r, p, Ap, d, st, nullptr}, ws, s, &fin, &on_chip));
     if (on_chip == Onchip::kAborted) VCLHIP_TRY(start());
   }
   if (on_chip == Onchip::kDone) {
@@ -1819,7 +1819,7 @@ __global__ __launch_bounds__(kBlock) void mixed1_update_kernel(uint32_t n, float
   const float beta = static_cast<float>(st->beta);
   const uint32_t lw = xcd_logical_block();
   uint32_t c0, c1;
-  chunk_range_w(n, W, lw, gridDim.x, c0, c1);
+  cg_vec_rows(n, lw, c0, c1);
   double acc[2] = {0, 0};
   for_packs<W>(c0, c1, [&](uint32_t i, auto w) {
     constexpr int V = decltype(w)::value;
@@ -1859,9 +1859,9 @@ __global__ __launch_bounds__(kBlock) void mixed1_iter_kernel(KState* __restrict_
 {
   if (st->flags & (kFlagDone | kFlagPause)) return;
   double sums[4];
-  block_sum_partials_k<4, double>({slot_ptr(part, kSlotRZ), slot_ptr(part, kSlotRR), slot_ptr(part, kSlotApAp),
-                                   slot_ptr(part, kSlotPAp)},
-                                  {g_vec, Jac ? g_vec : 0u, g_prod, g_prod}, sums);
+  owner_sums_k<4, double>({slot_ptr(part, kSlotRZ), slot_ptr(part, kSlotRR), slot_ptr(part, kSlotApAp),
+                           slot_ptr(part, kSlotPAp)},
+                          {g_vec, Jac ? g_vec : 0u, g_prod, g_prod}, sums);
   const double rz = sums[0];
   const double rr = Jac ? sums[1] : rz;
   const double ApAp = sums[2], pAp = sums[3];
@@ -2293,32 +2293,34 @@ static int mixed_cg_solve(const M* A, const float* values32, const double* b, do
     VCLHIP_TRY(ws.alloc(&zc, 1));
     VCLHIP_TRY(jacobi_diag(op32, d32, zc, s));
   }
-  KState h;
-  init_state(h, P, hist);
-  h.inner_tol = P->inner_tol;
-  VCLHIP_TRY(upload_state(st, h, s));
-
-  const uint32_t gv = solver_vec_grid(n);
+  const uint32_t gv = cg_vec_chunks(n);
   const bool v4 = aligned16({b, x});
-  if (jac)
-    VCLHIP_LAUNCH_W(v4, (mixed_init_kernel<true, 4>), (mixed_init_kernel<true, 1>), gv, s, n, b, x, x32, r32, p32, d32,
-                    part);
-  else
-    VCLHIP_LAUNCH_W(v4, (mixed_init_kernel<false, 4>), (mixed_init_kernel<false, 1>), gv, s, n, b, x, x32, r32, p32,
-                    d32, part);
-  VCLHIP_TRY(check_launch("mixed_init_kernel"));
-  if (mode == 1) {
+  auto start = [&]() -> int {
+    KState h;
+    init_state(h, P, hist);
+    h.inner_tol = P->inner_tol;
+    VCLHIP_TRY(upload_state(st, h, s));
     if (jac)
-      op32.launch(s, p32, EpiCg<float, true>{Ap32, p32, d32}, slot_ptr(part, kSlotApAp), nullptr, 0u);
+      VCLHIP_LAUNCH_W(v4, (mixed_init_kernel<true, 4>), (mixed_init_kernel<true, 1>), gv, s, n, b, x, x32, r32, p32,
+                      d32, part);
     else
-      op32.launch(s, p32, EpiCg<float, false>{Ap32, p32, d32}, slot_ptr(part, kSlotApAp), nullptr, 0u);
-    VCLHIP_TRY(check_launch("mixed prod"));
-  }
-  if (jac)
-    hipLaunchKernelGGL(mixed_setup_kernel<true>, dim3(1), dim3(kBlock), 0, s, st, part, gv, op32.grid, mode);
-  else
-    hipLaunchKernelGGL(mixed_setup_kernel<false>, dim3(1), dim3(kBlock), 0, s, st, part, gv, op32.grid, mode);
-  VCLHIP_TRY(check_launch("mixed_setup_kernel"));
+      VCLHIP_LAUNCH_W(v4, (mixed_init_kernel<false, 4>), (mixed_init_kernel<false, 1>), gv, s, n, b, x, x32, r32, p32,
+                      d32, part);
+    VCLHIP_TRY(check_launch("mixed_init_kernel"));
+    if (mode == 1) {
+      if (jac)
+        op32.launch(s, p32, EpiCg<float, true>{Ap32, p32, d32}, slot_ptr(part, kSlotApAp), nullptr, 0u);
+      else
+        op32.launch(s, p32, EpiCg<float, false>{Ap32, p32, d32}, slot_ptr(part, kSlotApAp), nullptr, 0u);
+      VCLHIP_TRY(check_launch("mixed prod"));
+    }
+    if (jac)
+      hipLaunchKernelGGL(mixed_setup_kernel<true>, dim3(1), dim3(kBlock), 0, s, st, part, gv, op32.grid, mode);
+    else
+      hipLaunchKernelGGL(mixed_setup_kernel<false>, dim3(1), dim3(kBlock), 0, s, st, part, gv, op32.grid, mode);
+    return check_launch("mixed_setup_kernel");
+  };
+  VCLHIP_TRY(start());
 
   uint32_t* flags = &st->flags;
   const uint32_t run_mask = kFlagDone | kFlagPause;
@@ -2369,9 +2371,18 @@ static int mixed_cg_solve(const M* A, const float* values32, const double* b, do
     return check_launch("mixed CG correction");
   };
   KState fin;
-  VCLHIP_TRY(run_iterations(
-      s, st, 0u, P->max_iters, P, x, launch_iter, [](uint32_t) { return false; }, [](uint32_t) { return 0; }, fin,
-      false, tail));
+  // The inner iterations between two corrections in one launch where the FP32 vectors fit the chip, with
+  // the same results (variant 1: one launch per step).
+  Onchip on_chip = Onchip::kNo;
+  if (mode == 1 && !jac && inner_is_dia && op32.grid == cg_prod_chunks(n) && P->variant != 1 && !P->use_graph &&
+      !P->monitor) {
+    VCLHIP_TRY(onchip_cg<float>({n, op32.dia, false, true, x32, r32, p32, Ap32, nullptr, st, tail}, ws, s, &fin, &on_chip));
+    if (on_chip == Onchip::kAborted) VCLHIP_TRY(start());
+  }
+  if (on_chip != Onchip::kDone)
+    VCLHIP_TRY(run_iterations(
+        s, st, 0u, P->max_iters, P, x, launch_iter, [](uint32_t) { return false; }, [](uint32_t) { return 0; }, fin,
+        false, tail));
   R->iters = fin.iter;
   R->error = fin.nrs > 0 ? std::sqrt(fin.res / fin.nrs) : 0.0;
   R->restarts = fin.updates;

@@ -30,6 +30,10 @@
 // 128^3 runs 19 us (47 us with three): 7 for the product, whose far rows come from L2, 2 for storing
 // p, 7 waiting for the workgroups at the XCDs' edges, whose far rows come from further away.
 //
+// The mixed solver runs its FP32 inner iterations between two FP64 corrections the same way, up to 16
+// rows a lane: 160^3 variable coefficients 36 us an iteration (55 us with three launches), of which the
+// FP32 values, 115 MB read from the Infinity Cache, are the larger part.
+//
 // Every sum is formed in the order of the kernel-per-step modes (cg_sums.hpp), so the results are
 // theirs bit for bit.
 //
@@ -176,6 +180,7 @@ __host__ __device__ inline OcPart oc_part(uint32_t n, uint32_t gp, uint32_t m, u
 template <typename T>
 struct OcArgs {
   uint32_t n, nd, gp, m, nwg;
+  uint32_t mixed;   // the mixed solver's inner iteration: its end test
   uint32_t far;     // halo form: mask of the diagonals read from memory (the first and the last)
   uint32_t ext;     // LDS entries for p
   uint32_t reach;   // halo form: workgroups on each side that own reached rows
@@ -268,7 +273,7 @@ __global__ __launch_bounds__(kOcThreads) void onchip_cg_kernel(OcArgs<T> a)
   __shared__ uint32_t ok;
 
   KState* const st = a.st;
-  if ((st->flags & kFlagDone) != 0 || ld_agent(a.abort) != 0) return;
+  if ((st->flags & (kFlagDone | kFlagPause)) != 0 || ld_agent(a.abort) != 0) return;
   const uint32_t iter0 = st->iter;
   // workgroups of one XCD take neighbouring rows: what they exchange then stays in its L2
   const uint32_t w = gridDim.x % 8 == 0 ? xcd_logical_block() : blockIdx.x;
@@ -346,7 +351,10 @@ __global__ __launch_bounds__(kOcThreads) void onchip_cg_kernel(OcArgs<T> a)
 #pragma unroll
   for (int s = 0; s < NC; ++s) codes[s] = 0;
 #pragma unroll
-  for (uint32_t i = 0; i < ND; ++i) one[i] = Val == kValOne && dia[i] != kAbsent ? a.table[dia[i] * kDiaCodes + 1] : T(0);
+  for (uint32_t i = 0; i < ND; ++i) {
+    one[i] = Val == kValOne && dia[i] != kAbsent ? a.table[dia[i] * kDiaCodes + 1] : T(0);
+    if (!(one[i] > 0 || one[i] < 0)) one[i] = T(0);  // zero and NaN are not there
+  }
 #pragma unroll
   for (int c = 0; c < CPV; ++c)
 #pragma unroll
@@ -368,7 +376,8 @@ __global__ __launch_bounds__(kOcThreads) void onchip_cg_kernel(OcArgs<T> a)
             const uint32_t at = dia[i] * n + row;
             if constexpr (Val == kValRegs) v[s][i] = a.code ? a.table[dia[i] * kDiaCodes + bcode.load(at)] : bval.load(at);
             if constexpr (Val == kValCodes) codes[s] |= static_cast<uint32_t>(bcode.load(at)) << (4 * i);
-            if constexpr (Val == kValOne) codes[s / 4] |= static_cast<uint32_t>(bcode.load(at)) << (8 * (s % 4) + i);
+            if constexpr (Val == kValOne)
+              codes[s / 4] |= (one[i] != T(0) ? static_cast<uint32_t>(bcode.load(at)) : 0u) << (8 * (s % 4) + i);
           }
       }
     }
@@ -413,6 +422,7 @@ __global__ __launch_bounds__(kOcThreads) void onchip_cg_kernel(OcArgs<T> a)
     }
   }
 
+  const double rr_stop = static_cast<double>(st->inner_tol) * st->rr_ref;
   const double nrs = st->nrs, tol2 = st->tol * st->tol, atol2 = st->abs_tol * st->abs_tol;
   const uint32_t max_iters = st->max_iters;
   double alpha = st->alpha, beta = st->beta;
@@ -595,7 +605,7 @@ __global__ __launch_bounds__(kOcThreads) void onchip_cg_kernel(OcArgs<T> a)
               xv = lp[delta[i] + l];
             }
             T val;
-            uint32_t there;  // all bits where the entry is there (no stored value of the operator is zero or NaN)
+            uint32_t there;  // all bits where the entry is there
             if constexpr (Val == kValOne) {
               val = one[i];
               there = static_cast<uint32_t>(static_cast<int32_t>(codes[s / 4] << (31 - (8 * (s % 4) + i))) >> 31);
@@ -603,9 +613,9 @@ __global__ __launch_bounds__(kOcThreads) void onchip_cg_kernel(OcArgs<T> a)
               if constexpr (Val == kValRegs) val = v[s][i];
               if constexpr (Val == kValCodes) val = stab[i * kDiaCodes + (codes[s] >> (4 * i) & 15u)];
               if constexpr (Val == kValStream) val = vv[c][i];
-              there = val != T(0) ? ~0u : 0u;
+              there = __builtin_islessgreater(val, T(0)) ? ~0u : 0u;  // not zero, not NaN
             }
-            sum += masked(xv, there) * val;  // an absent entry adds a zero, whatever xv is
+            sum += masked(xv * val, there);  // an absent entry adds a zero, whatever xv is
           }
           // the next tiles', while this one's sums go on
           if constexpr (Val == kValStream)
@@ -702,20 +712,27 @@ __global__ __launch_bounds__(kOcThreads) void onchip_cg_kernel(OcArgs<T> a)
     const double pAp = (tot[2][0] + tot[2][1]) + (tot[2][2] + tot[2][3]);
 
     // ---- cg_iter_kernel's step (cg.hpp:170-180)
-    const bool conv = uniform(fabs(rr / nrs) < tol2 || fabs(rr) < atol2);
+    // mixed1_iter_kernel's end test asks for an FP64 correction
+    const bool conv = uniform(a.mixed ? rr < rr_stop || rr / nrs < tol2 : fabs(rr / nrs) < tol2 || fabs(rr) < atol2);
     const bool done = conv || iter >= max_iters;
     alpha = uniform(rr / pAp);
     beta = uniform((alpha * alpha * ApAp - rr) / rr);
-    more = !done && k + 1 == kOcSlice;  // the next launch goes on from here
+    // the vectors are needed again: by the next launch, or by the correction
+    more = done ? a.mixed != 0 : k + 1 == kOcSlice;
     if (w == 0 && tid == 0) {
       record_history(st, iter, rr);
       if (done || more) {
         st->iter = iter;
         st->rr = rr;
+        st->rr2 = rr;
         st->alpha = alpha;
         st->beta = beta;
-        st->converged = conv ? 1u : 0u;
-        if (done) st->flags |= kFlagDone;
+        if (done && a.mixed) {
+          st->flags = (st->flags | kFlagPause) & ~kFlagNoPause;
+        } else {
+          st->converged = conv ? 1u : 0u;
+          if (done) st->flags |= kFlagDone;
+        }
       }
     }
     if (done || more) break;
@@ -780,6 +797,8 @@ void (*oc_kernel(bool ghost, int cpv, int tpc, uint32_t ghosts, OcVal how))(OcAr
   }
   if (cpv <= 2 && tpc <= 2) return oc_value_kernel<T, ND, Jac, W, 2, 0>(how);
   if (cpv <= 2 && tpc <= 4) return oc_value_kernel<T, ND, Jac, W, 4, 0>(how);
+  if constexpr (sizeof(T) == 4)
+    if (cpv <= 2 && tpc <= 8) return oc_value_kernel<T, ND, Jac, W, 8, 0>(how);
   return nullptr;
 }
 
@@ -804,7 +823,7 @@ bool oc_plan(const OnchipCg<T>& c, OcPlan<T>& pl)
   const OcVal how = !c.dia.code ? kValStream : (c.dia.distinct == 1 ? kValOne : kValCodes);
   const size_t tab = how == kValCodes ? kOcDiags * kDiaCodes * sizeof(T) : 0;
   // LDS entries after the workgroup's own that the lanes without a row read
-  const size_t spare = 4 * kBlock;
+  const size_t spare = 8 * kBlock;
   int32_t reach_rows = 0;
   for (uint32_t i = 0; i < nd; ++i) reach_rows = std::max(reach_rows, std::abs(c.dia.first_off[i]));
   // the LDS entries of a full workgroup: no workgroup has more
@@ -877,6 +896,7 @@ int onchip_cg(const OnchipCg<T>& c, Workspace& ws, hipStream_t s, KState* fin, O
   VCLHIP_TRY(vclhip_fill_zero(sh, sizeof(Shared), s));
   OcArgs<T> a{};
   a.n = c.n;
+  a.mixed = c.after ? 1u : 0u;
   a.nd = c.dia.nd;
   a.gp = cg_prod_chunks(c.n);
   a.m = pl.m;
@@ -903,6 +923,7 @@ int onchip_cg(const OnchipCg<T>& c, Workspace& ws, hipStream_t s, KState* fin, O
   do {
     hipLaunchKernelGGL(pl.kernel, dim3(pl.nwg), dim3(kOcThreads), pl.lds, s, a);
     VCLHIP_TRY(check_launch("onchip_cg_kernel"));
+    if (c.after) VCLHIP_TRY(c.after());
     VCLHIP_HIP(hipMemcpyAsync(fin, c.st, sizeof(KState), hipMemcpyDeviceToHost, s));
     VCLHIP_HIP(hipStreamSynchronize(s));
     a.wait_first = a.wait;

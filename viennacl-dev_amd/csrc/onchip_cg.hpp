@@ -2,6 +2,8 @@
 // registers and LDS of the CUs and only boundary rows and inner products travel between them.
 #pragma once
 
+#include <functional>
+
 #include "krylov_state.hpp"
 #include "solver.hpp"
 
@@ -21,6 +23,9 @@ struct OnchipCg {
   T* Ap;
   const T* d;
   KState* st;
+  // The mixed solver: enqueues the FP64 correction, whose kernels return at once unless the iterations
+  // ended asking for one.  The solve then goes on until the correction says that it is done.
+  std::function<int()> after;
 };
 
 enum class Onchip { kNo, kDone, kAborted };
