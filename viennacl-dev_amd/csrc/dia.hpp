@@ -28,84 +28,152 @@ constexpr uint32_t kDiaDictSlots = kDiaCodes - 1;   // distinct values per diago
 constexpr uint32_t kDiaCodedMinRows = 1u << 18;      // a value dictionary only where bytes bound the product
 constexpr uint32_t kDiaDictGroups = 256;             // workgroups per diagonal collecting its values
 
+// What the detection passes tell the host.
+struct DiaFound {
+  uint32_t overflow;          // not a DIA candidate
+  uint32_t refuse;            // the fill met a row or value that the copy cannot stand for
+  uint32_t distinct;          // values in the longest table of the dictionary
+  uint32_t count;             // distinct offsets
+  uint32_t keys[kDiaMax];     // the first of them, as col - row + n, in no order
+};
+
+constexpr uint32_t kDiaBatch = 8;  // entries of a row whose loads are in flight together
+
 // Marks every offset col - row of the matrix in a bitmap (bit col - row + n).  A workgroup first
 // collects the distinct offsets of its 256 rows in an LDS hash table, so that the global bitmap
 // sees one atomic OR per distinct offset and workgroup; a workgroup whose rows hold more distinct
-// offsets than the table, or a column outside the square matrix, raises *overflow (the matrix is
-// then not a DIA candidate).
-template <typename I>
-__global__ __launch_bounds__(kBlock) void dia_offsets_kernel(const I* __restrict__ rp, const I* __restrict__ col,
-                                                             uint32_t n, unsigned long long* __restrict__ bits,
-                                                             uint32_t* __restrict__ overflow)
+// offsets than the table, or a column outside the square matrix, raises found->overflow (the matrix
+// is then not a DIA candidate).  Almost every look finds its offset: the table and the bitmap are read
+// before the atomics, which all lanes (all workgroups) would send to the same few words.  The 7-point
+// operator on 128^3: 196 us with the atomics alone and an entry at a time, 61 us now.
+static __global__ __launch_bounds__(kBlock) void dia_offsets_kernel(const uint32_t* __restrict__ rp,
+                                                                    const uint32_t* __restrict__ col, uint32_t n,
+                                                                    unsigned long long* bits, DiaFound* found)
 {
   __shared__ uint32_t keys[kDiaHash];
-  __shared__ volatile uint32_t full;
+  __shared__ uint32_t full;
   const uint32_t tid = threadIdx.x;
   for (uint32_t i = tid; i < kDiaHash; i += kBlock) keys[i] = 0;
   if (tid == 0) full = 0;
   __syncthreads();
   const uint32_t row = blockIdx.x * kBlock + tid;
+  bool many = false;
   if (row < n) {
     const uint32_t e1 = rp[row + 1];
-    for (uint32_t e = rp[row]; e < e1 && !full; ++e) {  // once the table is full the answer is known
-      const uint32_t c = col[e];
-      if (c >= n) {  // not a square-matrix column: no DIA copy
-        full = 1;
-        break;
+    for (uint32_t e = rp[row]; e < e1 && !many; e += kDiaBatch) {
+      uint32_t c[kDiaBatch];
+#pragma unroll
+      for (uint32_t j = 0; j < kDiaBatch; ++j) c[j] = col[e + j < e1 ? e + j : e1 - 1];
+#pragma unroll
+      for (uint32_t j = 0; j < kDiaBatch; ++j) {
+        if (c[j] >= n) many = true;  // not a square-matrix column: no DIA copy
+        const uint32_t key = c[j] + n - row;  // in [1, 2n - 1]; 0 marks an empty slot
+        uint32_t h = (key * 2654435761u) >> 25;
+        uint32_t probe = many ? kDiaMax + 1 : 0;
+        // kDiaMax + 1 occupied slots in a row mean more than kDiaMax distinct offsets: not a candidate
+        for (; probe <= kDiaMax; ++probe) {
+          uint32_t prev = __hip_atomic_load(&keys[h], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+          if (prev == 0u) prev = atomicCAS(&keys[h], 0u, key);
+          if (prev == 0u || prev == key) break;
+          h = (h + 1) & (kDiaHash - 1);
+        }
+        if (probe > kDiaMax) many = true;
       }
-      const uint32_t key = c + n - row;  // in [1, 2n - 1]; 0 marks an empty slot
-      uint32_t h = (key * 2654435761u) >> 25;
-      uint32_t probe = 0;
-      // kDiaMax + 1 occupied slots in a row mean more than kDiaMax distinct offsets: not a candidate
-      for (; probe <= kDiaMax; ++probe) {
-        const uint32_t prev = atomicCAS(&keys[h], 0u, key);
-        if (prev == 0u || prev == key) break;
-        h = (h + 1) & (kDiaHash - 1);
-      }
-      if (probe > kDiaMax) full = 1;
     }
   }
+  if (many) full = 1;
   __syncthreads();
   for (uint32_t i = tid; i < kDiaHash; i += kBlock) {
     const uint32_t k = keys[i];
-    if (k) atomicOr(&bits[k >> 6], 1ull << (k & 63));
+    if (k) {
+      const unsigned long long bit = 1ull << (k & 63);
+      if (!(__hip_atomic_load(&bits[k >> 6], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & bit)) atomicOr(&bits[k >> 6], bit);
+    }
   }
-  if (tid == 0 && full) *overflow = 1u;
+  if (tid == 0 && full) found->overflow = 1u;
 }
 
-// val[d * n + row] = A(row, row + off[d]) converted to T (val zeroed before); off ascending,
-// nd <= kDiaMax, and every offset of the matrix is in off.  A row whose columns do not strictly
-// increase (unsorted, or an entry given twice) raises *refuse: its sum in column order would not be
-// the CSR kernel's, and a repeated entry would be lost.  With `exact`, so does a stored value that
-// the DIA kernel would skip (a zero of either sign, or NaN): the CSR kernel multiplies every stored
-// entry, so 0 * Inf or a NaN value would reach its sum and not the DIA one.
-template <typename S, typename T>
+// Lists the bits of the map in found->keys (the first kDiaMax of them) and counts them.
+static __global__ __launch_bounds__(kBlock) void dia_list_kernel(const unsigned long long* __restrict__ bits,
+                                                                 uint32_t words, DiaFound* found)
+{
+  const uint32_t w = blockIdx.x * kBlock + threadIdx.x;
+  if (w >= words || found->overflow) return;
+  for (unsigned long long b = bits[w]; b; b &= b - 1) {
+    if (__hip_atomic_load(&found->count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) > kDiaMax) return;
+    const uint32_t i = atomicAdd(&found->count, 1u);
+    if (i < kDiaMax) found->keys[i] = w * 64 + static_cast<uint32_t>(__builtin_ctzll(b));
+  }
+}
+
+// val[d * n + row] = A(row, row + off[d]) converted to T, zero where the row has no such entry; off
+// ascending, nd <= kDiaMax, and every offset of the matrix is in off (`first` holds the first
+// kDiaGroup of them; Few: there are no more).  A row whose columns do not strictly increase
+// (unsorted, or an entry given twice) raises found->refuse: its sum in column order would not be the
+// CSR kernel's, and a repeated entry would be lost.  With `exact`, so does a stored value that the DIA
+// kernel would skip (a zero of either sign, or NaN): the CSR kernel multiplies every stored entry, so
+// 0 * Inf or a NaN value would reach its sum and not the DIA one.
+// Bound by its traffic (the CSR arrays once, the values once).  128^3, 7-point: 135 us and 18 us for a
+// pass of zeros before it, an entry at a time; 79 us with the loads of a batch in flight together.
+struct DiaFirstOffsets {
+  int32_t off[kDiaGroup];
+};
+
+template <typename S, typename T, bool Few>
 __global__ __launch_bounds__(kBlock) void dia_fill_kernel(const uint32_t* __restrict__ rp,
                                                           const uint32_t* __restrict__ col, const S* __restrict__ a,
-                                                          uint32_t n, const int32_t* __restrict__ off, uint32_t nd,
-                                                          int exact, T* __restrict__ val, uint32_t* __restrict__ refuse)
+                                                          uint32_t n, const int32_t* __restrict__ off,
+                                                          DiaFirstOffsets first, uint32_t nd, int exact,
+                                                          T* __restrict__ val, DiaFound* __restrict__ found)
 {
-  __shared__ int32_t so[kDiaMax];
-  if (threadIdx.x < nd) so[threadIdx.x] = off[threadIdx.x];
-  __syncthreads();
+  __shared__ int32_t so[Few ? 1 : kDiaMax];
+  if constexpr (!Few) {
+    if (threadIdx.x < nd) so[threadIdx.x] = off[threadIdx.x];
+    __syncthreads();
+  }
   const uint32_t row = blockIdx.x * kBlock + threadIdx.x;
   if (row >= n) return;
   const uint32_t e0 = rp[row], e1 = rp[row + 1];
-  for (uint32_t e = e0; e < e1; ++e) {
-    if (e > e0 && col[e] <= col[e - 1]) *refuse = 1u;
-    const S v = a[e];
-    if (exact && !(v > S(0) || v < S(0))) *refuse = 1u;
-    const int32_t o = static_cast<int32_t>(col[e] - row);
-    uint32_t lo = 0, hi = nd;
-    while (hi - lo > 1) {
-      const uint32_t mid = (lo + hi) / 2;
-      if (so[mid] <= o)
-        lo = mid;
-      else
-        hi = mid;
+  uint32_t have = 0, prev = 0;
+  bool bad = false;
+  for (uint32_t e = e0; e < e1; e += kDiaBatch) {
+    uint32_t c[kDiaBatch];
+    S v[kDiaBatch];
+#pragma unroll
+    for (uint32_t j = 0; j < kDiaBatch; ++j) {
+      const uint32_t at = e + j < e1 ? e + j : e1 - 1;
+      c[j] = col[at];
+      v[j] = a[at];
     }
-    val[static_cast<size_t>(lo) * n + row] = static_cast<T>(v);
+#pragma unroll
+    for (uint32_t j = 0; j < kDiaBatch; ++j) {
+      if (e + j < e1) {
+        if (e + j > e0 && c[j] <= prev) bad = true;
+        prev = c[j];
+        if (exact && !(v[j] > S(0) || v[j] < S(0))) bad = true;
+        const int32_t o = static_cast<int32_t>(c[j] - row);
+        uint32_t lo = 0;
+        if constexpr (Few) {
+#pragma unroll
+          for (uint32_t k = 1; k < kDiaGroup; ++k) lo += k < nd && first.off[k] <= o ? 1u : 0u;
+        } else {
+          uint32_t hi = nd;
+          while (hi - lo > 1) {
+            const uint32_t mid = (lo + hi) / 2;
+            if (so[mid] <= o)
+              lo = mid;
+            else
+              hi = mid;
+          }
+        }
+        val[static_cast<size_t>(lo) * n + row] = static_cast<T>(v[j]);
+        have |= 1u << lo;
+      }
+    }
   }
+  for (uint32_t d = 0; d < nd; ++d)
+    if (!(have >> d & 1u)) val[static_cast<size_t>(d) * n + row] = T(0);
+  if (bad) found->refuse = 1u;
 }
 
 // ---- value dictionaries: one table of at most kDiaDictSlots distinct values per diagonal.
@@ -237,36 +305,41 @@ inline size_t dia_code_bytes(uint32_t n, uint32_t nd)
   return (static_cast<size_t>(nd) * kDiaCodes * sizeof(T) + 255) / 256 * 256 + static_cast<size_t>(nd) * n;
 }
 
-// Builds the value dictionary of `dia` into `extra` (dia_code_bytes<T> bytes); *coded tells
-// whether every diagonal fit.  Temporaries come from `ws`; without them there is no dictionary.
+// Builds the value dictionary's tables of `dia` at `extra` (dia_code_bytes<T> bytes) and leaves the
+// length of the longest in found->distinct (past kDiaDictSlots: no dictionary).  Temporaries come from
+// `ws`; *keys stays null without them.
 template <typename T>
-static int build_dia_codes(DiaDev<T>& dia, void* extra, Workspace& ws, uint32_t* flag, hipStream_t s, bool* coded)
+static int build_dia_tables(const DiaDev<T>& dia, void* extra, Workspace& ws, DiaFound* found, hipStream_t s,
+                            unsigned long long** keys)
 {
-  *coded = false;
   const uint32_t n = dia.n_rows, nd = dia.nd;
   const uint32_t groups = std::min<uint32_t>(kDiaDictGroups, (n + kBlock - 1) / kBlock);
-  unsigned long long *sets, *keys;
-  if (!ws.try_alloc(&sets, static_cast<size_t>(nd) * groups * kDiaDictSlots) ||
-      !ws.try_alloc(&keys, static_cast<size_t>(nd) * kDiaCodes))
+  unsigned long long *sets, *k;
+  *keys = nullptr;
+  if (!ws.try_alloc(&sets, static_cast<size_t>(nd) * groups * kDiaDictSlots + static_cast<size_t>(nd) * kDiaCodes))
     return VCLHIP_SUCCESS;
-  T* table = static_cast<T*>(extra);
-  uint8_t* code = static_cast<uint8_t*>(extra) + (static_cast<size_t>(nd) * kDiaCodes * sizeof(T) + 255) / 256 * 256;
-  VCLHIP_TRY(vclhip_fill_zero(flag, sizeof(uint32_t), s));
-  hipLaunchKernelGGL(dia_dict_collect_kernel<T>, dim3(groups, nd), dim3(kBlock), 0, s, dia.val, n, sets, flag);
+  k = sets + static_cast<size_t>(nd) * groups * kDiaDictSlots;
+  hipLaunchKernelGGL(dia_dict_collect_kernel<T>, dim3(groups, nd), dim3(kBlock), 0, s, dia.val, n, sets,
+                     &found->distinct);
   VCLHIP_TRY(check_launch("dia_dict_collect_kernel"));
-  hipLaunchKernelGGL(dia_dict_merge_kernel<T>, dim3(nd), dim3(kBlock), 0, s, sets, groups, table, keys, flag);
-  VCLHIP_TRY(check_launch("dia_dict_merge_kernel"));
-  uint32_t distinct = 0;
-  VCLHIP_HIP(hipMemcpyAsync(&distinct, flag, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-  VCLHIP_HIP(hipStreamSynchronize(s));
-  if (distinct > kDiaDictSlots) return VCLHIP_SUCCESS;
+  hipLaunchKernelGGL(dia_dict_merge_kernel<T>, dim3(nd), dim3(kBlock), 0, s, sets, groups, static_cast<T*>(extra), k,
+                     &found->distinct);
+  *keys = k;
+  return check_launch("dia_dict_merge_kernel");
+}
+
+// The codes behind the tables.
+template <typename T>
+static int build_dia_codes(DiaDev<T>& dia, void* extra, const unsigned long long* keys, uint32_t distinct, hipStream_t s)
+{
+  const uint32_t n = dia.n_rows, nd = dia.nd;
+  uint8_t* code = static_cast<uint8_t*>(extra) + (static_cast<size_t>(nd) * kDiaCodes * sizeof(T) + 255) / 256 * 256;
   hipLaunchKernelGGL(dia_encode_kernel<T>, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, dia.val, n, nd, keys,
                      code);
   VCLHIP_TRY(check_launch("dia_encode_kernel"));
   dia.code = code;
-  dia.table = table;
+  dia.table = static_cast<const T*>(extra);
   dia.distinct = distinct;
-  *coded = true;
   return VCLHIP_SUCCESS;
 }
 
@@ -292,29 +365,24 @@ static int build_dia(const vclhip_csr* A, Workspace& ws, hipStream_t s, double m
   if (n == 0 || A->n_cols != n || n >= (1u << 30) || !A->row_ptr || !A->col_idx || !A->values)
     return VCLHIP_SUCCESS;
   if (static_cast<uint64_t>(A->nnz) > static_cast<uint64_t>(kDiaMax) * n) return VCLHIP_SUCCESS;
-  const size_t words = (2ull * n + 64) / 64;
-  unsigned long long* bits;
-  uint32_t* overflow;
-  if (!ws.try_alloc(&bits, words) || !ws.try_alloc(&overflow, 1)) return VCLHIP_SUCCESS;
+  const uint32_t words = static_cast<uint32_t>((2ull * n + 64) / 64);
+  unsigned long long* bits;  // the map, then the record
+  constexpr uint32_t kRecord = (sizeof(DiaFound) + 7) / 8;
+  if (!ws.try_alloc(&bits, words + kRecord)) return VCLHIP_SUCCESS;
+  DiaFound* found = reinterpret_cast<DiaFound*>(bits + words);
   const uint32_t g = (n + kBlock - 1) / kBlock;
-  VCLHIP_TRY(vclhip_fill_zero(bits, words * sizeof(unsigned long long), s));
-  VCLHIP_TRY(vclhip_fill_zero(overflow, sizeof(uint32_t), s));
-  hipLaunchKernelGGL(dia_offsets_kernel<uint32_t>, dim3(g), dim3(kBlock), 0, s, A->row_ptr, A->col_idx, n, bits,
-                     overflow);
+  VCLHIP_TRY(vclhip_fill_zero(bits, (words + kRecord) * sizeof(unsigned long long), s));
+  hipLaunchKernelGGL(dia_offsets_kernel, dim3(g), dim3(kBlock), 0, s, A->row_ptr, A->col_idx, n, bits, found);
   VCLHIP_TRY(check_launch("dia_offsets_kernel"));
-  std::vector<unsigned long long> hb(words);
-  uint32_t hover = 0;
-  VCLHIP_HIP(hipMemcpyAsync(hb.data(), bits, words * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
-  VCLHIP_HIP(hipMemcpyAsync(&hover, overflow, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+  hipLaunchKernelGGL(dia_list_kernel, dim3((words + kBlock - 1) / kBlock), dim3(kBlock), 0, s, bits, words, found);
+  VCLHIP_TRY(check_launch("dia_list_kernel"));
+  DiaFound hf;
+  VCLHIP_HIP(hipMemcpyAsync(&hf, found, sizeof(DiaFound), hipMemcpyDeviceToHost, s));
   VCLHIP_HIP(hipStreamSynchronize(s));
-  if (hover) return VCLHIP_SUCCESS;
+  if (hf.overflow || hf.count > kDiaMax) return VCLHIP_SUCCESS;
   std::vector<int32_t> offs;
-  for (size_t w = 0; w < words; ++w)
-    for (unsigned long long b = hb[w]; b; b &= b - 1) {
-      if (offs.size() == kDiaMax) return VCLHIP_SUCCESS;
-      const uint64_t k = w * 64 + static_cast<uint64_t>(__builtin_ctzll(b));
-      offs.push_back(static_cast<int32_t>(static_cast<int64_t>(k) - n));
-    }
+  for (uint32_t i = 0; i < hf.count; ++i) offs.push_back(static_cast<int32_t>(static_cast<int64_t>(hf.keys[i]) - n));
+  std::sort(offs.begin(), offs.end());
   const uint32_t nd = static_cast<uint32_t>(offs.size());
   if (nd == 0 || static_cast<double>(nd) * n > max_fill * static_cast<double>(A->nnz)) return VCLHIP_SUCCESS;
   const size_t vbytes = static_cast<size_t>(nd) * n * sizeof(T);
@@ -330,25 +398,26 @@ static int build_dia(const vclhip_csr* A, Workspace& ws, hipStream_t s, double m
   }
   T* val = static_cast<T*>(arr.val);
   VCLHIP_HIP(hipMemcpyAsync(arr.off, offs.data(), nd * sizeof(int32_t), hipMemcpyHostToDevice, s));
-  VCLHIP_TRY(vclhip_fill_zero(val, vbytes, s));
-  VCLHIP_TRY(vclhip_fill_zero(overflow, sizeof(uint32_t), s));  // reused as the refusal flag
-  hipLaunchKernelGGL((dia_fill_kernel<S, T>), dim3(g), dim3(kBlock), 0, s, A->row_ptr, A->col_idx,
-                     static_cast<const S*>(A->values), n, arr.off, nd, exact ? 1 : 0, val, overflow);
+  DiaFirstOffsets first{};
+  for (uint32_t i = 0; i < nd && i < kDiaGroup; ++i) first.off[i] = offs[i];
+  auto fill = nd <= kDiaGroup ? dia_fill_kernel<S, T, true> : dia_fill_kernel<S, T, false>;
+  hipLaunchKernelGGL(fill, dim3(g), dim3(kBlock), 0, s, A->row_ptr, A->col_idx, static_cast<const S*>(A->values), n,
+                     arr.off, first, nd, exact ? 1 : 0, val, found);
   VCLHIP_TRY(check_launch("dia_fill_kernel"));
-  VCLHIP_HIP(hipMemcpyAsync(&hover, overflow, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+  DiaDev<T> made{};
+  made.val = val;
+  made.off = arr.off;
+  made.n_rows = n;
+  made.nd = nd;
+  for (uint32_t i = 0; i < kDiaGroup; ++i) made.first_off[i] = first.off[i];
+  unsigned long long* keys = nullptr;
+  void* extra = static_cast<char*>(arr.val) + vpad;
+  if (try_codes) VCLHIP_TRY(build_dia_tables<T>(made, extra, ws, found, s, &keys));
+  VCLHIP_HIP(hipMemcpyAsync(&hf, found, sizeof(DiaFound), hipMemcpyDeviceToHost, s));
   VCLHIP_HIP(hipStreamSynchronize(s));  // offs lives on the host stack
-  if (hover) return VCLHIP_SUCCESS;
-  out->val = val;
-  out->off = arr.off;
-  for (uint32_t i = 0; i < nd && i < kDiaGroup; ++i) out->first_off[i] = offs[i];
-  out->n_rows = n;
-  out->nd = nd;
-  out->code = nullptr;
-  out->table = nullptr;
-  if (try_codes) {
-    bool coded = false;
-    VCLHIP_TRY(build_dia_codes<T>(*out, static_cast<char*>(arr.val) + vpad, ws, overflow, s, &coded));
-  }
+  if (hf.refuse) return VCLHIP_SUCCESS;
+  if (keys && hf.distinct <= kDiaDictSlots) VCLHIP_TRY(build_dia_codes<T>(made, extra, keys, hf.distinct, s));
+  *out = made;
   *built = true;
   return VCLHIP_SUCCESS;
 }
