@@ -2,6 +2,7 @@
 // streams and events.
 #include <cstring>
 #include <mutex>
+#include <utility>
 #include <vector>
 
 #include "device.hpp"
@@ -32,6 +33,49 @@ int device_cu_count()
     cache[dev] = cu;
   }
   return cache[dev];
+}
+
+// The device's workspace pool; null where pools are not to be had.
+static hipMemPool_t workspace_pool()
+{
+  static std::mutex mu;
+  static std::vector<std::pair<bool, hipMemPool_t> > pools;
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0) return nullptr;
+  std::lock_guard<std::mutex> lock(mu);
+  if (static_cast<int>(pools.size()) <= dev) pools.resize(dev + 1, {false, nullptr});
+  auto& slot = pools[dev];
+  if (!slot.first) {
+    slot.first = true;
+    hipMemPoolProps props{};
+    props.allocType = hipMemAllocationTypePinned;
+    props.location.type = hipMemLocationTypeDevice;
+    props.location.id = dev;
+    uint64_t keep = kPoolKeep;
+    if (hipMemPoolCreate(&slot.second, &props) != hipSuccess ||
+        hipMemPoolSetAttribute(slot.second, hipMemPoolAttrReleaseThreshold, &keep) != hipSuccess) {
+      (void)hipGetLastError();
+      slot.second = nullptr;
+    }
+  }
+  return slot.second;
+}
+
+hipError_t workspace_malloc(void** p, size_t bytes, hipStream_t s)
+{
+  const hipMemPool_t pool = workspace_pool();
+  if (!pool) return hipMallocAsync(p, bytes, s);
+  hipError_t e = hipMallocFromPoolAsync(p, bytes, pool, s);
+  if (e == hipSuccess) return e;
+  (void)hipGetLastError();
+  workspace_trim();
+  return hipMallocFromPoolAsync(p, bytes, pool, s);
+}
+
+void workspace_trim()
+{
+  const hipMemPool_t pool = workspace_pool();
+  if (pool && hipMemPoolTrimTo(pool, 0) != hipSuccess) (void)hipGetLastError();
 }
 
 __global__ __launch_bounds__(kBlock) void fill_bytes_kernel(uint8_t* __restrict__ p, size_t bytes)
@@ -119,6 +163,9 @@ int vclhip_malloc(void** ptr, size_t bytes)
   if (!ptr) return vclhip::invalid("ptr is NULL");
   *ptr = nullptr;
   if (bytes == 0) return VCLHIP_SUCCESS;
+  if (hipMalloc(ptr, bytes) == hipSuccess) return VCLHIP_SUCCESS;
+  (void)hipGetLastError();
+  vclhip::workspace_trim();  // what the solvers' pool keeps may be what is missing
   VCLHIP_HIP(hipMalloc(ptr, bytes));
   return VCLHIP_SUCCESS;
 }

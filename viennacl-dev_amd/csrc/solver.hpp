@@ -273,8 +273,10 @@ class SolveStream {
 
 // ------------------------------------------------------------------ device workspace
 
-// Stream-ordered allocations released when the object goes out of scope; or, made over an arena
-// (a caller's device buffer), 256-byte aligned pieces of that buffer and no allocation at all.
+// Stream-ordered memory (workspace_malloc) released when the object goes out of scope, handed out in
+// 256-byte aligned pieces of slabs of at least kSlab bytes: a solve makes 10 to 20 small allocations,
+// at about 10 us each.  Or, made over an arena (a caller's device buffer), pieces of that buffer and no
+// allocation at all.
 class Workspace {
  public:
   explicit Workspace(hipStream_t s) : s_(s) {}
@@ -293,10 +295,7 @@ class Workspace {
       }
       return VCLHIP_SUCCESS;
     }
-    void* v = nullptr;
-    VCLHIP_HIP(hipMallocAsync(&v, count * sizeof(U) + 256, s_));
-    ptrs_.push_back(v);
-    *p = static_cast<U*>(v);
+    VCLHIP_HIP(get(p, count));
     return VCLHIP_SUCCESS;
   }
   // For optional buffers: false (and the HIP error cleared) when the allocation fails.
@@ -304,15 +303,10 @@ class Workspace {
   bool try_alloc(U** p, size_t count)
   {
     if (arena_) return take(p, count);
-    void* v = nullptr;
-    if (hipMallocAsync(&v, count * sizeof(U) + 256, s_) != hipSuccess || !v) {
-      (void)hipGetLastError();
-      *p = nullptr;
-      return false;
-    }
-    ptrs_.push_back(v);
-    *p = static_cast<U*>(v);
-    return true;
+    if (get(p, count) == hipSuccess) return true;
+    (void)hipGetLastError();
+    *p = nullptr;
+    return false;
   }
   // Bytes still free in the arena (no limit without one).
   size_t arena_left() const { return arena_ ? cap_ - used_ : ~size_t(0); }
@@ -321,6 +315,35 @@ class Workspace {
   static size_t arena_bytes(size_t elem, size_t count) { return (elem * count + 256 + 255) & ~size_t(255); }
 
  private:
+  static constexpr size_t kSlab = size_t(8) << 20;
+
+  template <typename U>
+  hipError_t get(U** p, size_t count)
+  {
+    const size_t bytes = arena_bytes(sizeof(U), count);
+    if (bytes > slab_left_) {
+      void* v = nullptr;
+      size_t size = bytes < kSlab ? kSlab : bytes;
+      hipError_t e = workspace_malloc(&v, size, s_);
+      if (e != hipSuccess && size > bytes) {
+        size = bytes;
+        e = workspace_malloc(&v, size, s_);
+      }
+      if (e != hipSuccess) return e;
+      ptrs_.push_back(v);
+      if (size - bytes < slab_left_) {  // the rest of the slab in use is the larger one: keep it
+        *p = static_cast<U*>(v);
+        return hipSuccess;
+      }
+      slab_ = static_cast<char*>(v);
+      slab_left_ = size;
+    }
+    *p = reinterpret_cast<U*>(slab_);
+    slab_ += bytes;
+    slab_left_ -= bytes;
+    return hipSuccess;
+  }
+
   template <typename U>
   bool take(U** p, size_t count)
   {
@@ -336,6 +359,8 @@ class Workspace {
 
   hipStream_t s_;
   std::vector<void*> ptrs_;
+  char* slab_ = nullptr;  // what is left of the newest slab
+  size_t slab_left_ = 0;
   char* arena_ = nullptr;  // 256-byte aligned
   size_t cap_ = 0, used_ = 0;
 };
