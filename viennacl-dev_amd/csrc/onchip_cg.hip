@@ -23,7 +23,9 @@
 // iteration, and 6.3 with neighbours on different XCDs.
 // The operator's values stay in registers (small systems), or as one bit per entry where every
 // diagonal has one value (the constant-coefficient Laplacians), as packed 4-bit codes into value
-// tables in LDS, or are read again in every iteration (they then come from the caches).
+// tables in LDS, or as stored: as many diagonals as fit in LDS, the others read again in every iteration
+// (Jacobi-CG on 97 x 83 x 71, whose 32 MB of values come to just the L2s' size: 20 us an iteration with
+// all of them read, 12 with six of seven diagonals in LDS).
 //
 // What bounds it: 256^2 runs 4.5 us an iteration, of which the exchange of the sums takes 1.6 and the
 // wait for the stored A p and the workgroup's own sums 1.0 (7.4 us with one launch per iteration);
@@ -69,8 +71,11 @@ constexpr uint32_t kOcSlice = 4096;             // iterations of a launch at mos
 static_assert(kOcSlice % 2 == 0, "a launch ends with A p in ex1");
 
 // Where the operator's values are: in registers; as 4-bit codes in registers, the tables in LDS; as one
-// bit per entry in registers, one value per diagonal; or read in every iteration.
-enum OcVal { kValRegs = 0, kValCodes = 1, kValStream = 2, kValOne = 3 };
+// bit per entry in registers, one value per diagonal; or as stored, read in every iteration, but for
+// the first half of the diagonals or all but the last, which LDS holds.
+enum OcVal { kValRegs = 0, kValCodes = 1, kValStream = 2, kValOne = 3, kValHalf = 4, kValMost = 5 };
+constexpr bool val_stored(OcVal v) { return v == kValStream || v == kValHalf || v == kValMost; }
+constexpr uint32_t val_held(OcVal v, uint32_t nd) { return v == kValMost ? nd - 1 : (v == kValHalf ? nd / 2 : 0); }
 
 // Relaxed accesses at agent scope: single-location coherence between the XCDs.
 template <typename U>
@@ -290,6 +295,8 @@ __global__ __launch_bounds__(kOcThreads) void onchip_cg_kernel(OcArgs<T> a)
   T* const stab = reinterpret_cast<T*>(oc_lds);
   T* const lp = stab + (Val == kValCodes ? kOcDiags * kDiaCodes : 0u);
   T* const lsq = lp + a.ext;
+  T* const lv = lsq + rows;  // [slot][row] of the values held
+  constexpr uint32_t kHeld = val_held(Val, ND);
 
   if (tid == 0) {
     ok = 1;
@@ -371,9 +378,13 @@ __global__ __launch_bounds__(kOcThreads) void onchip_cg_kernel(OcArgs<T> a)
         ap[s] = bex1.load(row);
         lp[own + l] = bp.load(row);
 #pragma unroll
+        for (uint32_t i = 0; i < kHeld; ++i) lv[i * rows + l] = T(0);
+#pragma unroll
         for (uint32_t i = 0; i < ND; ++i)
           if (dia[i] != kAbsent && row < n) {
             const uint32_t at = dia[i] * n + row;
+            if constexpr (kHeld > 0)
+              if (i < kHeld) lv[i * rows + l] = bval.load(at);
             if constexpr (Val == kValRegs) v[s][i] = a.code ? a.table[dia[i] * kDiaCodes + bcode.load(at)] : bval.load(at);
             if constexpr (Val == kValCodes) codes[s] |= static_cast<uint32_t>(bcode.load(at)) << (4 * i);
             if constexpr (Val == kValOne)
@@ -519,14 +530,15 @@ __global__ __launch_bounds__(kOcThreads) void onchip_cg_kernel(OcArgs<T> a)
     }
 
     // the first tiles' values, on their way during the waits
-    T vv[Val == kValStream ? CPV : 1][ND];
+    T vv[val_stored(Val) ? CPV : 1][ND - kHeld];
     auto load_values = [&](int c, int j) {
       const uint32_t row = lo + first[c] + j * kBlock;
       const bool here = static_cast<uint32_t>(j) < cnt[c] && row < n;
 #pragma unroll
-      for (uint32_t i = 0; i < ND; ++i) vv[c][i] = bval.load(here && dia[i] != kAbsent ? dia[i] * n + row : kOcNowhere);
+      for (uint32_t i = kHeld; i < ND; ++i)
+        vv[c][i - kHeld] = bval.load(here && dia[i] != kAbsent ? dia[i] * n + row : kOcNowhere);
     };
-    if constexpr (Val == kValStream)
+    if constexpr (val_stored(Val))
 #pragma unroll
       for (int c = 0; c < CPV; ++c) load_values(c, 0);
 
@@ -612,13 +624,18 @@ __global__ __launch_bounds__(kOcThreads) void onchip_cg_kernel(OcArgs<T> a)
             } else {
               if constexpr (Val == kValRegs) val = v[s][i];
               if constexpr (Val == kValCodes) val = stab[i * kDiaCodes + (codes[s] >> (4 * i) & 15u)];
-              if constexpr (Val == kValStream) val = vv[c][i];
+              if constexpr (val_stored(Val)) {
+                if (i < kHeld)
+                  val = lv[i * rows + l];
+                else
+                  val = vv[c][i - kHeld];
+              }
               there = __builtin_islessgreater(val, T(0)) ? ~0u : 0u;  // not zero, not NaN
             }
             sum += masked(xv * val, there);  // an absent entry adds a zero, whatever xv is
           }
           // the next tiles', while this one's sums go on
-          if constexpr (Val == kValStream)
+          if constexpr (val_stored(Val))
             if (j + 1 < TPC) load_values(c, j + 1);
           if constexpr (Ghosts == 0)
             if (j + kAhead < TPC) load_far(c, j + kAhead);
@@ -782,6 +799,10 @@ void (*oc_value_kernel(OcVal how))(OcArgs<T>)
 {
   if (how == kValOne) return onchip_cg_kernel<T, ND, Jac, W, 2, TPC, kValOne, Ghosts>;
   if (how == kValCodes) return onchip_cg_kernel<T, ND, Jac, W, 2, TPC, kValCodes, Ghosts>;
+  if constexpr (TPC == 2) {  // more rows than that leave LDS no room
+    if (how == kValMost) return onchip_cg_kernel<T, ND, Jac, W, 2, TPC, kValMost, Ghosts>;
+    if (how == kValHalf) return onchip_cg_kernel<T, ND, Jac, W, 2, TPC, kValHalf, Ghosts>;
+  }
   return onchip_cg_kernel<T, ND, Jac, W, 2, TPC, kValStream, Ghosts>;
 }
 
@@ -820,10 +841,9 @@ bool oc_plan(const OnchipCg<T>& c, OcPlan<T>& pl)
   const int tpc = static_cast<int>((tiles + gp - 1) / gp);
   auto wg_tiles = [&](bool up) { return static_cast<uint32_t>((static_cast<uint64_t>(tiles) * chunks + (up ? gp - 1 : 0)) / gp); };
   const uint32_t rows = wg_tiles(true) * kBlock;
-  const OcVal how = !c.dia.code ? kValStream : (c.dia.distinct == 1 ? kValOne : kValCodes);
-  const size_t tab = how == kValCodes ? kOcDiags * kDiaCodes * sizeof(T) : 0;
-  // LDS entries after the workgroup's own that the lanes without a row read
-  const size_t spare = 8 * kBlock;
+  const size_t tab = c.dia.code && c.dia.distinct != 1 ? kOcDiags * kDiaCodes * sizeof(T) : 0;
+  const uint32_t slots = nd <= 5 ? 5 : 7;
+  const uint32_t spare = (tpc <= 1 ? 1u : tpc <= 2 ? 2u : tpc <= 4 ? 4u : 8u) * kBlock;  // that lanes without a row read past the end
   int32_t reach_rows = 0;
   for (uint32_t i = 0; i < nd; ++i) reach_rows = std::max(reach_rows, std::abs(c.dia.first_off[i]));
   // the LDS entries of a full workgroup: no workgroup has more
@@ -834,7 +854,13 @@ bool oc_plan(const OnchipCg<T>& c, OcPlan<T>& pl)
   };
   auto pick = [&](bool ghost, uint32_t far) {
     const uint32_t ext = segments(far);
-    const size_t bytes = tab + (static_cast<size_t>(ext) + std::max<size_t>(rows, spare)) * sizeof(T);
+    auto lds_bytes = [&](OcVal how) {
+      return tab + (static_cast<size_t>(ext) + rows * (1 + val_held(how, slots)) + spare) * sizeof(T);
+    };
+    OcVal how = !c.dia.code ? kValStream : (c.dia.distinct == 1 ? kValOne : kValCodes);
+    if (how == kValStream && !ghost && tpc <= 2)
+      how = lds_bytes(kValMost) <= kOcLds ? kValMost : (lds_bytes(kValHalf) <= kOcLds ? kValHalf : kValStream);
+    const size_t bytes = lds_bytes(how);
     if (bytes > kOcLds) return false;
     if (!c.wide) return false;
     const uint32_t g = ext - rows;
@@ -843,7 +869,7 @@ bool oc_plan(const OnchipCg<T>& c, OcPlan<T>& pl)
       return c.jacobi ? oc_kernel<T, ND, true, kVecW<T> >(ghost, cpv, tpc, g, how)
                       : oc_kernel<T, ND, false, kVecW<T> >(ghost, cpv, tpc, g, how);
     };
-    void (*k)(OcArgs<T>) = nd <= 5 ? choose(std::integral_constant<uint32_t, 5>()) : choose(std::integral_constant<uint32_t, 7>());
+    void (*k)(OcArgs<T>) = slots == 5 ? choose(std::integral_constant<uint32_t, 5>()) : choose(std::integral_constant<uint32_t, 7>());
     if (!k) return false;
     pl.kernel = k;
     pl.ghost = ghost;
