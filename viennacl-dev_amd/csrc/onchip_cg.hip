@@ -27,10 +27,10 @@
 // (Jacobi-CG on 97 x 83 x 71, whose 32 MB of values come to just the L2s' size: 20 us an iteration with
 // all of them read, 12 with six of seven diagonals in LDS).
 //
-// What bounds it: 256^2 runs 4.5 us an iteration, of which the exchange of the sums takes 1.6 and the
-// wait for the stored A p and the workgroup's own sums 1.0 (7.4 us with one launch per iteration);
-// 128^3 runs 19 us (47 us with three): 7 for the product, whose far rows come from L2, 2 for storing
-// p, 7 waiting for the workgroups at the XCDs' edges, whose far rows come from further away.
+// What bounds it: 256^2 runs 3.9 us an iteration, of which the exchange of the sums takes 1.7 and the
+// workgroup's own sums 0.6 (7.4 us with one launch per iteration); 128^3 runs 18 us (47 us with three):
+// 7 for the product, whose far rows come from L2, 2 for storing p, 6 waiting for the workgroups at the
+// XCDs' edges, whose far rows come from further away.
 //
 // The mixed solver runs its FP32 inner iterations between two FP64 corrections the same way, up to 16
 // rows a lane: 160^3 variable coefficients 36 us an iteration (55 us with three launches), of which the
@@ -255,6 +255,20 @@ __device__ __forceinline__ T masked(T v, uint32_t mask)
   }
 }
 
+// The wavefront sums of three values (wave_sum's, bit for bit) in the lanes of rows 0, 1 and 2: each
+// step folds what is left of two values into one register, so that the last four steps run once
+// (23 instructions for 66).
+__device__ __forceinline__ double wave_sums3(double v0, double v1, double v2)
+{
+  swap_rows<32>(v0, v2);
+  v0 += v2;  // half 0: the first value's, half 1: the third's
+  double u = v1;
+  swap_rows<32>(v1, u);
+  v1 += u;
+  swap_rows<16>(v0, v1);
+  return row_sum(v0 + v1);
+}
+
 // Slot of ND holds a diagonal of the operator, in offset order with the last one in the last slot, or
 // nothing (a zero entry): the slots are a compile-time number, so that a row's loads and sums have no
 // branches.
@@ -290,7 +304,7 @@ __global__ __launch_bounds__(kOcThreads) void onchip_cg_kernel(OcArgs<T> a)
   const uint32_t lo = q.t0 * kBlock, rows = (q.t1 - q.t0) * kBlock;  // rows past the system's end are held as zeros
   const uint32_t mv = a.gp <= kOwners ? 1u : cg_vec_per_owner(n);
   const uint32_t v0 = a.gp <= kOwners ? q.o0 : q.o0 * mv;
-  const uint32_t nvec = (q.o1 - q.o0) * mv, nprod = q.p1 - q.p0;
+  const uint32_t nvec = (q.o1 - q.o0) * mv;
 
   T* const stab = reinterpret_cast<T*>(oc_lds);
   T* const lp = stab + (Val == kValCodes ? kOcDiags * kDiaCodes : 0u);
@@ -653,36 +667,28 @@ __global__ __launch_bounds__(kOcThreads) void onchip_cg_kernel(OcArgs<T> a)
 #pragma unroll
     for (int c = 0; c < CPV; ++c) {
       const uint32_t at = vb + static_cast<uint32_t>(c) * kOcBlocks;
-      const double sv = wave_sum(acc_v[c]), sa = wave_sum(acc_a[c]), sp = wave_sum(acc_p[c]);
-      if (lane == 0) {
-        red[0][at][wave] = sv;
-        red[1][at][wave] = sa;
-        red[2][at][wave] = sp;
-      }
+      const double sum = wave_sums3(acc_v[c], acc_a[c], acc_p[c]);
+      if ((lane & 15u) == 0 && lane < 16 * kOcSums) red[lane / 16][at][wave] = sum;
     }
     if constexpr (Ghosts > 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // A p is where the neighbours read it
     __syncthreads();
-    unsigned long long* const set = a.lines + (iter & 1u) * kOwners * kOcLine;
     if (tid < kWave) {
-      double part = 0;
-      if (rq < kOcSums && rc < (rq == 0 ? nvec : nprod)) {
-        part = red[rq][rc][0];
-#pragma unroll
-        for (int i = 1; i < kWavesPerBlock; ++i) part += red[rq][rc][i];
-      }
       double sum = 0;
 #pragma unroll
       for (uint32_t i = 0; i < CPV * kOcBlocks; ++i) {
-        const double u = __shfl(part, static_cast<int>((rq << 3) + ((own_b + i) & 7u)), kWave);
-        if (own_b + i < own_e) sum += u;
+        const double* const w4 = red[rq < kOcSums ? rq : 0][(own_b + i) & 7u];
+        double part = w4[0];
+#pragma unroll
+        for (int j = 1; j < kWavesPerBlock; ++j) part += w4[j];
+        if (own_b + i < own_e) sum += part;
       }
-      if (a.m >= 2) sum += __shfl_xor(sum, 1, kWave);
-      if (a.m >= 4) sum += __shfl_xor(sum, 2, kWave);
-      sum = __shfl(sum, static_cast<int>(((lane >> 1) & 7u) << 3), kWave);
-      if (lane < 2 * kOcSums) {
-        const unsigned long long bits = static_cast<unsigned long long>(__double_as_longlong(sum));
-        const unsigned long long half = (lane & 1u) ? bits >> 32 : bits & 0xffffffffull;
-        st_agent(set + w * kOcLine + lane, static_cast<unsigned long long>(iter) << 32 | half);
+      if (a.m >= 2) sum += dpp_move<kDppXor1>(sum);
+      if (a.m >= 4) sum += dpp_move<kDppXor2>(sum);
+      if (rc == 0 && rq < kOcSums) {
+        const unsigned long long bits = __builtin_bit_cast(unsigned long long, sum);
+        typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+        __builtin_amdgcn_raw_buffer_store_b128(u32x4{static_cast<uint32_t>(bits), iter, static_cast<uint32_t>(bits >> 32), iter},
+                                               line_rsrc, ((iter & 1u) * kOwners + w) * kOcLine * 8 + 16 * rq, 0, 16);
       }
     }
     // ---- everyone's sums, then the binary tree over them
