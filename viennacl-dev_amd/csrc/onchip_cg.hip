@@ -17,6 +17,9 @@
 //       reached rows are read from memory: a second, neighbours-only wait per iteration (about 1 us),
 //       but no ghost state.  With more than two rows a lane the ghosts' registers spill (100^3: 24 us
 //       an iteration as ghost, 11 as halo; Jacobi on 97 x 83 x 71: 30 and 20).
+// From 128 workgroups on, the first of each XCD adds up its XCD's sums and all others read those eight:
+// 256 workgroups that poll 256 lines hold each other up (exchange at 64^3 3.5 us, 2.4 in two steps;
+// CG on 128^3 9.5 -> 7.5 ms; with 128 workgroups both take 2.3 us, and 64 take 1.7 in one step).
 // Data that another workgroup reads is stored and loaded at agent scope, which the XCDs' L2s keep
 // coherent, and a wave waits for its stores before its workgroup publishes.  Workgroups of one XCD own
 // neighbouring rows, so that most of that stays in its L2: storing p of 128^3 takes 2.1 us an
@@ -28,8 +31,8 @@
 // all of them read, 12 with six of seven diagonals in LDS).
 //
 // What bounds it: 256^2 runs 3.9 us an iteration, of which the exchange of the sums takes 1.7 and the
-// workgroup's own sums 0.6 (7.4 us with one launch per iteration); 128^3 runs 18 us (47 us with three):
-// 7 for the product, whose far rows come from L2, 2 for storing p, 6 waiting for the workgroups at the
+// workgroup's own sums 0.6 (7.4 us with one launch per iteration); 128^3 runs 14 us (47 us with three):
+// 6 for the product, whose far rows come from L2, 2 for storing p, 3 waiting for the workgroups at the
 // XCDs' edges, whose far rows come from further away.
 //
 // The mixed solver runs its FP32 inner iterations between two FP64 corrections the same way, up to 16
@@ -65,6 +68,8 @@ constexpr uint32_t kOcDiags = 7;                // diagonals at most
 constexpr uint32_t kOcChunks = 8;               // chunks of a workgroup at most
 constexpr int kOcSums = 3;
 constexpr uint32_t kOcLine = 8;                 // 8-byte words of a workgroup's line
+constexpr uint32_t kXcds = 8;
+constexpr uint32_t kOcLines = kOwners + kXcds;  // lines of a set: the workgroups' and the XCDs'
 constexpr size_t kOcLds = 160 * 1024 - 2048;    // dynamic LDS at most (the static part stays below 2 KB)
 constexpr uint64_t kOcClock = 100;              // wall clock ticks per microsecond
 constexpr uint32_t kOcSlice = 4096;             // iterations of a launch at most: it then lets other work in
@@ -188,6 +193,7 @@ struct OcArgs {
   uint32_t mixed;   // the mixed solver's inner iteration: its end test
   uint32_t far;     // halo form: mask of the diagonals read from memory (the first and the last)
   uint32_t ext;     // LDS entries for p
+  uint32_t per_xcd; // workgroups that add up their sums before all others see them; 0: none do
   uint32_t reach;   // halo form: workgroups on each side that own reached rows
   int32_t off[kOcDiags];
   const T* val;
@@ -452,7 +458,7 @@ __global__ __launch_bounds__(kOcThreads) void onchip_cg_kernel(OcArgs<T> a)
   const uint32_t max_iters = st->max_iters;
   double alpha = st->alpha, beta = st->beta;
   const __amdgpu_buffer_rsrc_t line_rsrc =
-      __builtin_amdgcn_make_buffer_rsrc(a.lines, 0, 2 * kOwners * kOcLine * 8, 0x00027000);
+      __builtin_amdgcn_make_buffer_rsrc(a.lines, 0, 2 * kOcLines * kOcLine * 8, 0x00027000);
 
   bool more = false;
   for (uint32_t k = 0;; ++k) {
@@ -672,6 +678,7 @@ __global__ __launch_bounds__(kOcThreads) void onchip_cg_kernel(OcArgs<T> a)
     }
     if constexpr (Ghosts > 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // A p is where the neighbours read it
     __syncthreads();
+    const uint32_t set = (iter & 1u) * kOcLines;
     if (tid < kWave) {
       double sum = 0;
 #pragma unroll
@@ -688,40 +695,71 @@ __global__ __launch_bounds__(kOcThreads) void onchip_cg_kernel(OcArgs<T> a)
         const unsigned long long bits = __builtin_bit_cast(unsigned long long, sum);
         typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
         __builtin_amdgcn_raw_buffer_store_b128(u32x4{static_cast<uint32_t>(bits), iter, static_cast<uint32_t>(bits >> 32), iter},
-                                               line_rsrc, ((iter & 1u) * kOwners + w) * kOcLine * 8 + 16 * rq, 0, 16);
+                                               line_rsrc, (set + w) * kOcLine * 8 + 16 * rq, 0, 16);
       }
     }
     // ---- everyone's sums, then the binary tree over them
-    if (tid < kOwners) {
-      double s3[kOcSums] = {0, 0, 0};
-      if (tid < a.nwg) {
-        OcWait wait;
-        uint32_t word[4 * kOcSums];
-        for (;;) {
-          bool all = true;
+    auto read_line = [&](uint32_t line, double (&s3)[kOcSums]) {
+      OcWait wait;
+      uint32_t word[4 * kOcSums];
+      for (;;) {
+        bool all = true;
 #pragma unroll
-          for (int i = 0; i < kOcSums; ++i) {
-            typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-            const u32x4 b = __builtin_amdgcn_raw_buffer_load_b128(
-                line_rsrc, ((iter & 1u) * kOwners + tid) * kOcLine * 8 + 16 * i, 0, 16);
-            word[4 * i] = b.x;
-            word[4 * i + 1] = b.y;
-            word[4 * i + 2] = b.z;
-            word[4 * i + 3] = b.w;
-          }
-          asm volatile("" ::: "memory");
-#pragma unroll
-          for (int i = 0; i < 2 * kOcSums; ++i) all = all && word[2 * i + 1] == iter;
-          if (all) break;
-          if (!wait.again(a.abort, limit)) {
-            ok = 0;
-            break;
-          }
+        for (int i = 0; i < kOcSums; ++i) {
+          typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+          const u32x4 b = __builtin_amdgcn_raw_buffer_load_b128(line_rsrc, (set + line) * kOcLine * 8 + 16 * i, 0, 16);
+          word[4 * i] = b.x;
+          word[4 * i + 1] = b.y;
+          word[4 * i + 2] = b.z;
+          word[4 * i + 3] = b.w;
         }
+        asm volatile("" ::: "memory");
 #pragma unroll
-        for (int i = 0; i < kOcSums; ++i)
-          s3[i] = __longlong_as_double(static_cast<long long>(static_cast<unsigned long long>(word[4 * i + 2]) << 32 | word[4 * i]));
+        for (int i = 0; i < 2 * kOcSums; ++i) all = all && word[2 * i + 1] == iter;
+        if (all) break;
+        if (!wait.again(a.abort, limit)) {
+          ok = 0;
+          break;
+        }
       }
+#pragma unroll
+      for (int i = 0; i < kOcSums; ++i)
+        s3[i] = __longlong_as_double(static_cast<long long>(static_cast<unsigned long long>(word[4 * i + 2]) << 32 | word[4 * i]));
+    };
+    if (a.per_xcd != 0) {
+      // the subtree of an XCD's workgroups first, by the first of them; then the XCDs' sums
+      if (tid < kWave) {
+        double s3[kOcSums] = {0, 0, 0};
+        if (w % a.per_xcd == 0) {
+          if (lane < a.per_xcd) read_line(w + lane, s3);
+#pragma unroll
+          for (int i = 0; i < kOcSums; ++i) s3[i] = wave_tree(s3[i]);
+          if (lane < kOcSums) {
+            const double v = lane == 0 ? s3[0] : (lane == 1 ? s3[1] : s3[2]);
+            const unsigned long long bits = __builtin_bit_cast(unsigned long long, v);
+            typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+            __builtin_amdgcn_raw_buffer_store_b128(u32x4{static_cast<uint32_t>(bits), iter, static_cast<uint32_t>(bits >> 32), iter},
+                                                   line_rsrc, (set + kOwners + w / a.per_xcd) * kOcLine * 8 + 16 * lane, 0, 16);
+          }
+#pragma unroll
+          for (int i = 0; i < kOcSums; ++i) s3[i] = 0;
+        }
+        if (lane < kXcds) read_line(kOwners + lane, s3);
+#pragma unroll
+        for (int i = 0; i < kOcSums; ++i) {
+          s3[i] += dpp_move<kDppXor1>(s3[i]);
+          s3[i] += dpp_move<kDppXor2>(s3[i]);
+          s3[i] += dpp_move<kDppHalfMirror>(s3[i]);
+        }
+        if (lane < kOcSums) {
+          tot[lane][0] = lane == 0 ? s3[0] : (lane == 1 ? s3[1] : s3[2]);
+#pragma unroll
+          for (int i = 1; i < kWavesPerBlock; ++i) tot[lane][i] = 0;
+        }
+      }
+    } else if (tid < kOwners) {
+      double s3[kOcSums] = {0, 0, 0};
+      if (tid < a.nwg) read_line(tid, s3);
 #pragma unroll
       for (int i = 0; i < kOcSums; ++i) {
         s3[i] = wave_tree(s3[i]);
@@ -919,7 +957,7 @@ int onchip_cg(const OnchipCg<T>& c, Workspace& ws, hipStream_t s, KState* fin, O
   if (per_cu < 1) return VCLHIP_SUCCESS;
   // the exchange lines and the flags, cleared before the first launch
   struct Shared {
-    unsigned long long lines[2 * kOwners * kOcLine];
+    unsigned long long lines[2 * kOcLines * kOcLine];
     uint32_t flags[kOwners * 16];
   };
   Shared* sh;
@@ -933,6 +971,7 @@ int onchip_cg(const OnchipCg<T>& c, Workspace& ws, hipStream_t s, KState* fin, O
   a.gp = cg_prod_chunks(c.n);
   a.m = pl.m;
   a.nwg = pl.nwg;
+  a.per_xcd = pl.nwg >= 128 && pl.nwg % kXcds == 0 ? pl.nwg / kXcds : 0;
   a.far = pl.far;
   a.ext = pl.ext;
   a.reach = pl.reach;
