@@ -509,7 +509,8 @@ typedef struct vclhip_solver_result {
   uint32_t kernels_per_iter;  /* CG: kernels launched per iteration after the first (1 in fused mode,
                                  2 in compact mode, else 3; a solve that runs all iterations in one
                                  kernel reports the mode it would take otherwise); BiCGStab: 4 in compact mode, 6 pipelined,
-                                 8 with the reference's Jacobi recurrences; 0 from the other solvers */
+                                 8 with the reference's Jacobi recurrences (6 where the sums are few);
+                                 0 from the other solvers */
 } vclhip_solver_result;
 #define VCLHIP_USED_AS_GIVEN 0
 #define VCLHIP_USED_DIA 1

@@ -36,6 +36,10 @@ constexpr uint64_t kCompactPartialReads = 1ull << 20;
 // 11.0 against 12.0 at 518 K (350^2), even at 555-832 K (50^3, 392^2), 17.6 against 14.6 at 1.4 M
 // (450^2).
 constexpr uint64_t kFusedPartialReads = 1ull << 19;
+// BiCGStab with the reference's Jacobi recurrences: alpha and omega inside the vector kernels up to so
+// many partials read by all workgroups together, of the larger of the two sums (400 000 power-law rows,
+// 1.6 M reads: 52 us an iteration for 56; a scalar kernel takes 3.7 us and a launch).
+constexpr uint64_t kClassicPartialReads = 1ull << 21;
 
 // ------------------------------------------------------------------ epilogues
 
@@ -902,16 +906,54 @@ __global__ __launch_bounds__(kBlock) void bicgc_omega_kernel(KState* __restrict_
   st->omega = t1s / (nrm * nrm);
 }
 
-// x += alpha p + omega s; r = s - omega t1; partials <r,r>, <r,r0*>  (bicgstab.hpp:459-468)
+// s = r - alpha t0 with bicgc_alpha_kernel's alpha, which every workgroup forms itself from the
+// partial sums, in the same order; workgroup 0 stores it.
 template <typename T, int W>
+__global__ __launch_bounds__(kBlock) void bicgc_s_kernel(uint32_t n, T* __restrict__ s, const T* __restrict__ r,
+                                                         const T* __restrict__ t0, KState* __restrict__ st,
+                                                         const double* __restrict__ part, uint32_t g_prod)
+{
+  if (st->flags & kFlagDone) return;
+  const double t0r0 = block_sum_partials(slot_ptr(part, 2), g_prod);
+  const double a = st->rr / t0r0;
+  if (blockIdx.x == 0 && threadIdx.x == 0) st->alpha = a;
+  const T alpha = static_cast<T>(a);
+  const uint32_t lw = xcd_logical_block();
+  uint32_t c0, c1;
+  chunk_range_w(n, W, lw, gridDim.x, c0, c1);
+  for_packs<W>(c0, c1, [&](uint32_t i, auto w) {
+    constexpr int V = decltype(w)::value;
+    const Pack<V, T> vr = ldp<V>(r, i);
+    const Pack<V, T> va = ldp<V>(t0, i);
+    Pack<V, T> vs;
+#pragma unroll
+    for (int k = 0; k < V; ++k) vs.v[k] = vr.v[k] - alpha * va.v[k];
+    stp<V>(s, i, vs);
+  });
+}
+
+// x += alpha p + omega s; r = s - omega t1; partials <r,r>, <r,r0*>  (bicgstab.hpp:459-468).  Own: every
+// workgroup forms bicgc_omega_kernel's omega itself, as bicgc_s_kernel does alpha.
+template <typename T, int W, bool Own>
 __global__ __launch_bounds__(kBlock) void bicgc_xr_kernel(uint32_t n, T* __restrict__ x, const T* __restrict__ p,
                                                           const T* __restrict__ s, T* __restrict__ r,
                                                           const T* __restrict__ t1, const T* __restrict__ r0,
-                                                          const KState* __restrict__ st, double* __restrict__ part)
+                                                          KState* __restrict__ st, double* __restrict__ part,
+                                                          uint32_t g_prod)
 {
   if (st->flags & kFlagDone) return;
   const T alpha = static_cast<T>(st->alpha);
-  const T omega = static_cast<T>(st->omega);
+  double om;
+  if constexpr (Own) {
+    double sums[2];
+    block_sum_partials_k<2, double>({slot_ptr(part, 4), slot_ptr(part, 5)}, {g_prod, g_prod}, sums);
+    const double nrm = sqrt(sums[0]);
+    om = sums[1] / (nrm * nrm);
+    if (blockIdx.x == 0 && threadIdx.x == 0) st->omega = om;
+  } else {
+    om = st->omega;
+  }
+  const T omega = static_cast<T>(om);
   const uint32_t lw = xcd_logical_block();
   uint32_t c0, c1;
   chunk_range_w(n, W, lw, gridDim.x, c0, c1);
@@ -1537,16 +1579,28 @@ static int bicgstab_solve(const M* Ain, const T* b, T* x, int precond, const vcl
   const uint32_t stop_all = kFlagDone | kFlagFinishing;
   const int brk = jac ? 1 : 0;
   const bool classic = jac && P->variant == 0;
+  // alpha and omega inside the vector kernels (six kernels per iteration instead of eight) where all
+  // workgroups together read at most kClassicPartialReads partial sums for them
+  const bool fold = classic && 2ull * gv * op.grid <= kClassicPartialReads;
   auto launch_classic = [&]() -> int {
     // t0 = M^-1 A p -> Ap; alpha; s = r - alpha t0; t1 = M^-1 A s -> As; omega; x, r; test; p
     op.launch(s, p, EpiBicg<T, true, false>{Ap, p, r0, d}, slot_ptr(part, 2), flags, kFlagDone);
-    hipLaunchKernelGGL(bicgc_alpha_kernel, dim3(1), dim3(kBlock), 0, s, st, part, op.grid);
-    VCLHIP_LAUNCH_W(v2, (bicg_update_s_kernel<T, kVecW<T> >), (bicg_update_s_kernel<T, 1>), gv, s, n, sv, r, Ap, st,
-                    part);
+    if (fold) {
+      VCLHIP_LAUNCH_W(v2, (bicgc_s_kernel<T, kVecW<T> >), (bicgc_s_kernel<T, 1>), gv, s, n, sv, r, Ap, st, part, op.grid);
+    } else {
+      hipLaunchKernelGGL(bicgc_alpha_kernel, dim3(1), dim3(kBlock), 0, s, st, part, op.grid);
+      VCLHIP_LAUNCH_W(v2, (bicg_update_s_kernel<T, kVecW<T> >), (bicg_update_s_kernel<T, 1>), gv, s, n, sv, r, Ap, st,
+                      part);
+    }
     op.launch(s, sv, EpiBicg<T, true, true>{As, sv, r0, d}, slot_ptr(part, 4), flags, kFlagDone);
-    hipLaunchKernelGGL(bicgc_omega_kernel, dim3(1), dim3(kBlock), 0, s, st, part, op.grid);
-    VCLHIP_LAUNCH_W(v2, (bicgc_xr_kernel<T, kVecW<T> >), (bicgc_xr_kernel<T, 1>), gv, s, n, x, p, sv, r, As, r0, st,
-                    part);
+    if (fold) {
+      VCLHIP_LAUNCH_W(v2, (bicgc_xr_kernel<T, kVecW<T>, true>), (bicgc_xr_kernel<T, 1, true>), gv, s, n, x, p, sv, r,
+                      As, r0, st, part, op.grid);
+    } else {
+      hipLaunchKernelGGL(bicgc_omega_kernel, dim3(1), dim3(kBlock), 0, s, st, part, op.grid);
+      VCLHIP_LAUNCH_W(v2, (bicgc_xr_kernel<T, kVecW<T>, false>), (bicgc_xr_kernel<T, 1, false>), gv, s, n, x, p, sv, r,
+                      As, r0, st, part, op.grid);
+    }
     hipLaunchKernelGGL(bicgc_check_kernel, dim3(1), dim3(kBlock), 0, s, st, part, gv);
     VCLHIP_LAUNCH_W(v2, (bicgc_p_kernel<T, kVecW<T> >), (bicgc_p_kernel<T, 1>), gv, s, n, p, r, Ap, st);
     return check_launch("bicgstab iteration");
@@ -1621,7 +1675,7 @@ static int bicgstab_solve(const M* Ain, const T* b, T* x, int precond, const vcl
   R->restarts = restarts;
   R->converged = static_cast<int>(fin.converged);
   R->operator_used = used_dia;
-  R->kernels_per_iter = compact ? 4u : (classic ? 8u : 6u);
+  R->kernels_per_iter = compact ? 4u : (classic && !fold ? 8u : 6u);
   return copy_history(P, hist, fin.iter, s);
 }
 
