@@ -30,9 +30,9 @@ def band(n, offsets, values, seed=0):
 def run(vh, A, b, dtype, **kw):
     db, dx = vh.DeviceArray.from_numpy(b.astype(dtype)), vh.DeviceArray.zeros(b.size, dtype)
     hist = np.zeros(kw["max_iters"])
-    vh.lib().vclhip_onchip_last()
+    vh.lib().onchip_cg_last()
     res = vh.cg(A, db, dx, history=hist, **kw)
-    return dx.to_numpy(), res, hist, vh.lib().vclhip_onchip_last()
+    return dx.to_numpy(), res, hist, vh.lib().onchip_cg_last()
 
 
 def check(vh, A, b, dtype, want, **kw):
@@ -111,7 +111,7 @@ def test_values_that_are_not_finite(dev, vh):
 def test_gives_up_when_its_workgroups_do_not_meet(dev, vh):
     """With a wait limit of zero every first unsuccessful look gives up: the launched modes take over
     from the start, with their results."""
-    limit = vh.lib().vclhip_onchip_wait_limit
+    limit = vh.lib().onchip_cg_wait_limit
     limit.argtypes = [ctypes.c_double]
     for n, offsets in ((65536, [1, 256]), (700001, [1, 88, 7744])):
         rp, col, val = band(n, offsets, 1)
@@ -141,9 +141,9 @@ def test_mixed_inner_iterations(dev, vh, case):
     out = []
     for variant in (0, 1):
         db, dx, hist = vh.DeviceArray.from_numpy(b), vh.DeviceArray.zeros(n, np.float64), np.zeros(kw["max_iters"])
-        vh.lib().vclhip_onchip_last()
+        vh.lib().onchip_cg_last()
         res = vh.mixed_cg(A, db, dx, variant=variant, history=hist, **kw)
-        out.append((dx.to_numpy(), hist, res, vh.lib().vclhip_onchip_last()))
+        out.append((dx.to_numpy(), hist, res, vh.lib().onchip_cg_last()))
     (x0, h0, r0, m0), (x1, h1, r1, m1) = out
     assert (m0, m1) == (RAN, NOT_RUN)
     assert r0.iters == r1.iters and r0.restarts == r1.restarts and r0.error == r1.error and r0.converged == r1.converged

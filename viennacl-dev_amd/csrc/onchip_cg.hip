@@ -55,7 +55,7 @@
 
 namespace vclhip {
 
-// Hooks of the tests (vclhip_onchip_*, not part of the API), per thread: the wait limit in microseconds
+// Hooks of the tests (onchip_cg_wait_limit and onchip_cg_last, not part of the API), per thread: the wait limit in microseconds
 // (below zero: the usual ones), and whether the last CG solve ran here (1), gave up (2) or neither (0).
 static thread_local double t_wait_us = -1;
 static thread_local int t_on_chip = 0;
@@ -874,7 +874,7 @@ bool oc_plan(const OnchipCg<T>& c, OcPlan<T>& pl)
   if (nd == 0 || nd > kOcDiags || n >= (1u << 24)) return false;  // 32-bit byte offsets
   const uint32_t gp = cg_prod_chunks(n), tiles = cg_tiles(n);
   const uint32_t owners = gp < kOwners ? gp : kOwners;
-  // fewer workgroups exchange faster (2.3 us for 64, 2.4 for 128, 2.8 for 256), so small systems put
+  // fewer workgroups exchange faster (1.7 us for 64, 2.3 for 128, 2.4 for 256), so small systems put
   // several owners, one chunk or two each, on a workgroup's four 256-lane groups
   pl.m = gp <= kOwners ? 4u : (gp <= 2 * kOwners ? 2u : 1u);
   pl.nwg = (owners + pl.m - 1) / pl.m;
@@ -1011,13 +1011,13 @@ template int onchip_cg<float>(const OnchipCg<float>&, Workspace&, hipStream_t, K
 
 extern "C" {
 
-int vclhip_onchip_wait_limit(double microseconds)
+int onchip_cg_wait_limit(double microseconds)
 {
   vclhip::t_wait_us = microseconds;
   return VCLHIP_SUCCESS;
 }
 
-int vclhip_onchip_last(void)
+int onchip_cg_last(void)
 {
   const int v = vclhip::t_on_chip;
   vclhip::t_on_chip = 0;
