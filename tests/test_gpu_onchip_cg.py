@@ -56,6 +56,10 @@ CASES = {
     "regs_300001": (300001, [1, 547], 0, True), "halo_524289": (524289, [1, 80, 6400], 0, True),
     "halo_one_value": (700001, [1, 88, 7744], 1, True), "halo_codes": (700003, [1, 88, 7744], 3, True),
     "halo_wide": (1048577, [1, 101, 10201], 0, True), "halo_wide_one_value": (1500001, [1, 114, 13000], 1, True),
+    # a tile per chunk, unequal numbers of chunks per workgroup and a reach of many workgroups: the stencils
+    # of 1300 x 19 x 16, 1281 x 62 x 5, 1132 x 37 x 11 and 1568 x 63 x 4 (more workgroups than it waits for)
+    "unequal_stored": (395200, [1, 1300, 24700], 0, True), "unequal_one_value": (397110, [1, 1281, 79422], 1, True),
+    "unequal_codes": (460724, [1, 1132, 41884], 3, True), "unequal_too_far": (395136, [1, 1568, 98784], 0, False),
     "far_middle": (700001, [1, 7000, 7744], 1, False), "eight_diagonals": (70001, [1, 3, 40, 900], 0, False),
 }
 

@@ -55,8 +55,9 @@
 
 namespace vclhip {
 
-// Hooks of the tests (onchip_cg_wait_limit and onchip_cg_last, not part of the API), per thread: the wait limit in microseconds
-// (below zero: the usual ones), and whether the last CG solve ran here (1), gave up (2) or neither (0).
+// Hooks of the tests (onchip_cg_wait_limit, onchip_cg_last and onchip_cg_plan, not part of the API), per
+// thread: the wait limit in microseconds (below zero: the usual ones), and whether the last CG solve ran
+// here (1), gave up (2) or neither (0).
 static thread_local double t_wait_us = -1;
 static thread_local int t_on_chip = 0;
 
@@ -185,6 +186,33 @@ __host__ __device__ inline OcPart oc_part(uint32_t n, uint32_t gp, uint32_t m, u
   part_range(tiles, q.p0, gp, q.t0, unused);
   part_range(tiles, q.p1, gp, q.t1, unused);
   return q;
+}
+
+// For how many workgroups on each side one has to wait in the halo form: the farthest owner of a row
+// that its own rows reach along the diagonals (offsets ascending; the rows past the system's end count
+// as well, as they are loaded).  Walked over the workgroups themselves (at most 256): where the product
+// chunks are no multiple of the owners these hold unequal numbers of rows, and a bound from one of
+// their sizes is too short for others.
+inline uint32_t oc_reach(uint32_t n, uint32_t gp, uint32_t m, uint32_t nwg, uint32_t nd, const int32_t* off)
+{
+  uint32_t first[kOwners + 1] = {0};
+  for (uint32_t w = 0; w < nwg; ++w) {
+    const OcPart q = oc_part(n, gp, m, w);
+    first[w] = q.t0 * kBlock;
+    first[w + 1] = q.t1 * kBlock;
+  }
+  auto owner = [&](int64_t row) {
+    const int64_t r = std::min<int64_t>(std::max<int64_t>(row, 0), static_cast<int64_t>(n) - 1);
+    return static_cast<uint32_t>(std::upper_bound(first, first + nwg, static_cast<uint32_t>(r)) - first) - 1;
+  };
+  uint32_t reach = 0;
+  for (uint32_t w = 0; w < nwg; ++w) {
+    const uint32_t lo = owner(static_cast<int64_t>(first[w]) + off[0]);
+    const uint32_t hi = owner(static_cast<int64_t>(first[w + 1]) - 1 + off[nd - 1]);
+    if (lo < w) reach = std::max(reach, w - lo);
+    if (hi > w) reach = std::max(reach, hi - w);
+  }
+  return reach;
 }
 
 template <typename T>
@@ -868,7 +896,7 @@ void (*oc_kernel(bool ghost, int cpv, int tpc, uint32_t ghosts, OcVal how))(OcAr
 }
 
 template <typename T>
-bool oc_plan(const OnchipCg<T>& c, OcPlan<T>& pl)
+bool oc_plan(const OnchipCg<T>& c, uint32_t cus, OcPlan<T>& pl)
 {
   const uint32_t n = c.n, nd = c.dia.nd;
   if (nd == 0 || nd > kOcDiags || n >= (1u << 24)) return false;  // 32-bit byte offsets
@@ -878,18 +906,15 @@ bool oc_plan(const OnchipCg<T>& c, OcPlan<T>& pl)
   // several owners, one chunk or two each, on a workgroup's four 256-lane groups
   pl.m = gp <= kOwners ? 4u : (gp <= 2 * kOwners ? 2u : 1u);
   pl.nwg = (owners + pl.m - 1) / pl.m;
-  if (pl.nwg > static_cast<uint32_t>(device_cu_count())) return false;
+  if (pl.nwg > cus) return false;
   const uint32_t chunks = pl.m * ((gp + kOwners - 1) / kOwners);  // of a workgroup, at most
   const uint32_t vecs = pl.m * (gp <= kOwners ? 1u : cg_vec_per_owner(n));
   const int cpv = static_cast<int>((std::max(chunks, vecs) + kOcBlocks - 1) / kOcBlocks);
   const int tpc = static_cast<int>((tiles + gp - 1) / gp);
-  auto wg_tiles = [&](bool up) { return static_cast<uint32_t>((static_cast<uint64_t>(tiles) * chunks + (up ? gp - 1 : 0)) / gp); };
-  const uint32_t rows = wg_tiles(true) * kBlock;
+  const uint32_t rows = static_cast<uint32_t>((static_cast<uint64_t>(tiles) * chunks + gp - 1) / gp) * kBlock;  // at most
   const size_t tab = c.dia.code && c.dia.distinct != 1 ? kOcDiags * kDiaCodes * sizeof(T) : 0;
   const uint32_t slots = nd <= 5 ? 5 : 7;
   const uint32_t spare = (tpc <= 1 ? 1u : tpc <= 2 ? 2u : tpc <= 4 ? 4u : 8u) * kBlock;  // that lanes without a row read past the end
-  int32_t reach_rows = 0;
-  for (uint32_t i = 0; i < nd; ++i) reach_rows = std::max(reach_rows, std::abs(c.dia.first_off[i]));
   // the LDS entries of a full workgroup: no workgroup has more
   auto segments = [&](uint32_t far) {
     OcSegments g;
@@ -928,9 +953,7 @@ bool oc_plan(const OnchipCg<T>& c, OcPlan<T>& pl)
   for (uint32_t i = 1; i + 1 < nd; ++i)
     if (static_cast<uint32_t>(std::abs(c.dia.first_off[i])) >= rows) return false;
   const uint32_t far = 1u | 1u << (nd - 1);
-  const uint32_t least = wg_tiles(false) * kBlock;
-  if (least == 0) return false;
-  pl.reach = (static_cast<uint32_t>(reach_rows) + least - 1) / least + 1;
+  pl.reach = oc_reach(n, gp, pl.m, pl.nwg, nd, c.dia.first_off);
   if (2 * pl.reach + 1 > 2 * kWave) return false;
   return pick(false, far);
 }
@@ -943,7 +966,7 @@ int onchip_cg(const OnchipCg<T>& c, Workspace& ws, hipStream_t s, KState* fin, O
   *outcome = Onchip::kNo;
   t_on_chip = 0;
   OcPlan<T> pl;
-  if (!oc_plan(c, pl)) return VCLHIP_SUCCESS;
+  if (!oc_plan(c, static_cast<uint32_t>(device_cu_count()), pl)) return VCLHIP_SUCCESS;
   int dev = 0;
   VCLHIP_HIP(hipGetDevice(&dev));
   if (dev < 0 || dev >= 64) return VCLHIP_SUCCESS;
@@ -1004,6 +1027,29 @@ int onchip_cg(const OnchipCg<T>& c, Workspace& ws, hipStream_t s, KState* fin, O
   return VCLHIP_SUCCESS;
 }
 
+namespace {
+
+template <typename T>
+int oc_plan_of(OnchipCg<T> c, uint32_t cus, const int32_t* off, uint32_t distinct, uint32_t* reach, uint32_t* rows)
+{
+  static const uint8_t coded = 0;
+  c.dia.distinct = distinct;
+  c.dia.code = distinct ? &coded : nullptr;
+  std::copy(off, off + std::min(c.dia.nd, kDiaGroup), c.dia.first_off);
+  OcPlan<T> pl;
+  if (!oc_plan(c, cus, pl)) return 0;
+  const uint32_t gp = cg_prod_chunks(c.n);
+  for (uint32_t w = 0; w < pl.nwg; ++w) {
+    const OcPart q = oc_part(c.n, gp, pl.m, w);
+    rows[w] = q.t0 * kBlock;
+    rows[w + 1] = q.t1 * kBlock;
+  }
+  *reach = pl.ghost ? 0 : pl.reach;
+  return static_cast<int>(pl.nwg);
+}
+
+}  // namespace
+
 template int onchip_cg<double>(const OnchipCg<double>&, Workspace&, hipStream_t, KState*, Onchip*);
 template int onchip_cg<float>(const OnchipCg<float>&, Workspace&, hipStream_t, KState*, Onchip*);
 
@@ -1022,6 +1068,23 @@ int onchip_cg_last(void)
   const int v = vclhip::t_on_chip;
   vclhip::t_on_chip = 0;
   return v;
+}
+
+// The plan of an n-row system of nd diagonals (ascending offsets; `distinct` values on a diagonal, 0: as
+// stored) on a device of `cus` compute units, without one: the number of workgroups (0: not on chip),
+// the first row of each and the end of the last in rows[0 .. 256], and in *reach for how many workgroups
+// on each side it waits (0: the ghost form).
+int onchip_cg_plan(int single, int jacobi, uint32_t n, uint32_t nd, const int32_t* off, uint32_t distinct, uint32_t cus,
+                   uint32_t* reach, uint32_t* rows)
+{
+  if (single) {
+    vclhip::OnchipCg<float> c{};
+    c.n = n, c.dia.nd = nd, c.jacobi = jacobi != 0, c.wide = true;
+    return vclhip::oc_plan_of(c, cus, off, distinct, reach, rows);
+  }
+  vclhip::OnchipCg<double> c{};
+  c.n = n, c.dia.nd = nd, c.jacobi = jacobi != 0, c.wide = true;
+  return vclhip::oc_plan_of(c, cus, off, distinct, reach, rows);
 }
 
 }  // extern "C"
