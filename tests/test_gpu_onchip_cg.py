@@ -129,6 +129,26 @@ def test_gives_up_when_its_workgroups_do_not_meet(dev, vh):
         check(vh, A, b, np.float64, RAN, tol=1e-9, max_iters=400)
 
 
+@pytest.mark.parametrize("case", ["ghost", "halo"])
+def test_workgroups_that_start_after_others_gave_up(dev, vh, case):
+    """256 workgroups at a wait limit of zero, again and again: the first to look gives up while others
+    are still starting, which then leave at once, all waves of a workgroup together.  Every solve ends
+    and the launched modes take over with their results."""
+    limit = vh.lib().onchip_cg_wait_limit
+    limit.argtypes = [ctypes.c_double]
+    n, offsets, values = {"ghost": (300001, [1, 547], 0), "halo": (700001, [1, 88, 7744], 3)}[case]
+    rp, col, val = band(n, offsets, values, seed=n)
+    A, b = vh.CsrMatrix(rp, col, val), vh.random_uniform(3, n)
+    want, _, _, _ = run(vh, A, b, np.float64, variant=1, tol=1e-9, max_iters=40)
+    limit(0.0)
+    try:
+        for _ in range(25):
+            x, res, _, mode = run(vh, A, b, np.float64, tol=1e-9, max_iters=40)
+            assert mode == GAVE_UP and np.array_equal(x, want)
+    finally:
+        limit(-1.0)
+
+
 @pytest.mark.parametrize("case", ["diffusion_small", "diffusion_halo", "laplace_one_value", "sixteen_rows_a_lane", "limit"])
 def test_mixed_inner_iterations(dev, vh, case):
     """The mixed solver's FP32 inner iterations between two FP64 corrections in one launch: x, counts,

@@ -326,7 +326,6 @@ __global__ __launch_bounds__(kOcThreads) void onchip_cg_kernel(OcArgs<T> a)
   __shared__ uint32_t ok;
 
   KState* const st = a.st;
-  if ((st->flags & (kFlagDone | kFlagPause)) != 0 || ld_agent(a.abort) != 0) return;
   const uint32_t iter0 = st->iter;
   // workgroups of one XCD take neighbouring rows: what they exchange then stays in its L2
   const uint32_t w = gridDim.x % 8 == 0 ? xcd_logical_block() : blockIdx.x;
@@ -346,8 +345,11 @@ __global__ __launch_bounds__(kOcThreads) void onchip_cg_kernel(OcArgs<T> a)
   T* const lv = lsq + rows;  // [slot][row] of the values held
   constexpr uint32_t kHeld = val_held(Val, ND);
 
+  // Nothing to do, or others have given up before this workgroup started: one lane looks and all waves
+  // go by what it saw.  The abort word may be raised at any time, and waves that looked for themselves
+  // could part, some leaving and the rest going on without the sums and the waits of those.
   if (tid == 0) {
-    ok = 1;
+    ok = (st->flags & (kFlagDone | kFlagPause)) == 0 && ld_agent(a.abort) == 0 ? 1u : 0u;
     oc_segments(rows, nd, a.off, a.far, seg);
   }
   if constexpr (Val == kValCodes)
@@ -357,6 +359,7 @@ __global__ __launch_bounds__(kOcThreads) void onchip_cg_kernel(OcArgs<T> a)
     }
   for (uint32_t i = tid; i < a.ext; i += kOcThreads) lp[i] = T(0);
   __syncthreads();
+  if (!uniform(ok != 0)) return;
   const uint32_t own = __builtin_amdgcn_readfirstlane(seg.own);
   const uint32_t all_ghosts = __builtin_amdgcn_readfirstlane(seg.ext) - rows;
   uint32_t delta[ND], dia[ND];  // by slot
