@@ -149,6 +149,27 @@ def test_workgroups_that_start_after_others_gave_up(dev, vh, case):
         limit(-1.0)
 
 
+@pytest.mark.parametrize("precond", [0, 1])
+def test_solution_over_the_right_hand_side(dev, vh, precond):
+    """b and x in one array: the launched modes read b before they write x.  The one-launch solve gives the
+    same, and so does a solve that gives up and starts over in the launched modes."""
+    limit = vh.lib().onchip_cg_wait_limit
+    limit.argtypes = [ctypes.c_double]
+    rp, col, val = band(70001, [1, 265], 0)
+    A, b = vh.CsrMatrix(rp, col, val), vh.random_uniform(3, 70001)
+    kw = dict(precond=precond, tol=1e-9, max_iters=400)
+    want, _, _, _ = run(vh, A, b, np.float64, variant=1, **kw)
+    for microseconds, mode in ((-1.0, RAN), (0.0, GAVE_UP)):
+        x = vh.DeviceArray.from_numpy(b)
+        limit(microseconds)
+        try:
+            res = vh.cg(A, x, x, **kw)
+        finally:
+            limit(-1.0)
+        assert vh.lib().onchip_cg_last() == mode and res.converged
+        assert np.array_equal(x.to_numpy(), want)
+
+
 @pytest.mark.parametrize("case", ["diffusion_small", "diffusion_halo", "laplace_one_value", "sixteen_rows_a_lane", "limit"])
 def test_mixed_inner_iterations(dev, vh, case):
     """The mixed solver's FP32 inner iterations between two FP64 corrections in one launch: x, counts,

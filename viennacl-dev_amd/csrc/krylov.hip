@@ -1391,16 +1391,29 @@ static int cg_solve(const M* Ain, const T* b, T* x, int precond, const vclhip_so
   VCLHIP_TRY(dia_operator(op, ws, s, P, &used_dia));
   const uint32_t gv = cg_vec_chunks(n);
   const bool v2 = aligned16({b, x});  // workspace vectors are 256-byte aligned
+  // On-chip mode: all iterations in one launch where the vectors fit the CUs' registers and LDS, with
+  // the same results.  Not where the caller asks for a form of launches (graph, variant 1) or watches
+  // the iterations.  A solve that gives up starts over from b, so where x takes its place b is kept.
+  bool may_on_chip = op.fmt == OpFormat::Dia && op.grid == cg_prod_chunks(n) && P->variant == 0 && !P->use_graph && !P->monitor;
+  const T* rhs = b;
+  if (may_on_chip && b == x) {
+    T* kept;
+    may_on_chip = ws.try_alloc(&kept, n);
+    if (may_on_chip) {
+      VCLHIP_HIP(hipMemcpyAsync(kept, b, n * sizeof(T), hipMemcpyDeviceToDevice, s));
+      rhs = kept;
+    }
+  }
   // setup: x = 0, r = b, p = M^-1 b, Ap = A p, scalars
   auto start = [&]() -> int {
     KState h;
     init_state(h, P, hist);
     VCLHIP_TRY(upload_state(st, h, s));
     if (jac)
-      VCLHIP_LAUNCH_W(v2, (cg_init_kernel<T, true, kVecW<T> >), (cg_init_kernel<T, true, 1>), gv, s, n, b, x, r, p,
+      VCLHIP_LAUNCH_W(v2, (cg_init_kernel<T, true, kVecW<T> >), (cg_init_kernel<T, true, 1>), gv, s, n, rhs, x, r, p,
                       d, part);
     else
-      VCLHIP_LAUNCH_W(v2, (cg_init_kernel<T, false, kVecW<T> >), (cg_init_kernel<T, false, 1>), gv, s, n, b, x, r, p,
+      VCLHIP_LAUNCH_W(v2, (cg_init_kernel<T, false, kVecW<T> >), (cg_init_kernel<T, false, 1>), gv, s, n, rhs, x, r, p,
                       d, part);
     VCLHIP_TRY(check_launch("cg_init_kernel"));
     if (jac)
@@ -1484,11 +1497,8 @@ static int cg_solve(const M* Ain, const T* b, T* x, int precond, const vclhip_so
   };
   KState fin;
   const bool no_alloc = arena != nullptr;
-  // On-chip mode: all iterations in one launch where the vectors fit the CUs' registers and LDS, with
-  // the same results.  Not where the caller asks for a form of launches (graph, variant 1) or watches
-  // the iterations.
   Onchip on_chip = Onchip::kNo;
-  if (op.fmt == OpFormat::Dia && op.grid == cg_prod_chunks(n) && P->variant == 0 && !P->use_graph && !P->monitor) {
+  if (may_on_chip) {
     VCLHIP_TRY(onchip_cg<T>({n, op.dia, jac, v2, x, r, p, Ap, d, st, nullptr}, ws, s, &fin, &on_chip));
     if (on_chip == Onchip::kAborted) VCLHIP_TRY(start());
   }
