@@ -55,6 +55,12 @@ int vclhip_device_info(int device, char* name, size_t name_len, size_t* total_me
 int vclhip_malloc(void** ptr_dev, size_t bytes);
 /* handle deleter (backend/cuda.hpp:85-93) */
 int vclhip_free(void* ptr_dev);
+/* Solves take their device memory from a pool of the library's own, which keeps up to 512 MB per
+ * device for the next solve (no counterpart in the reference).  It goes back to the device when one
+ * of the library's own allocations would fail otherwise; this call gives back what the current
+ * device's pool keeps, for the caller's other allocators on the device.  Solves in progress keep
+ * what they use. */
+int vclhip_workspace_trim(void);
 /* memory_write (backend/memory.hpp:220-249 -> backend/cuda.hpp:154-177); returns when done */
 int vclhip_memcpy_h2d(void* dst_dev, const void* src_host, size_t bytes, void* stream);
 /* memory_read (backend/memory.hpp:261-292 -> backend/cuda.hpp:183-200); returns when done */

@@ -1,6 +1,7 @@
 """Host-side parts of libvclhip that need no GPU: the exported ABI, the CSR block planner,
 the generators and the project RNG."""
 import ctypes
+import re
 import subprocess
 
 import numpy as np
@@ -19,6 +20,16 @@ def test_library_exports_every_declared_symbol(vh):
     out = subprocess.run(["nm", "-D", "--defined-only", str(_abi.LIB_PATH)], capture_output=True, text=True).stdout
     exported = {line.split()[-1] for line in out.splitlines() if " T vclhip_" in line}
     assert set(declared) == exported
+
+
+def test_device_memory_comes_through_the_functions_that_trim(vh):
+    """The workspace pool keeps memory between solves, and gives it back before an allocation of the
+    library's fails: every allocation goes through the functions of runtime.hip that see to it."""
+    from vclhip import _abi
+    csrc = _abi.LIB_PATH.parent.parent / "csrc"
+    plain = re.compile(r"\bhip(Malloc|MallocAsync|MallocFromPoolAsync)\s*\(")
+    found = {f.name for f in csrc.iterdir() if f.suffix in (".hip", ".hpp", ".cpp") and plain.search(f.read_text())}
+    assert found == {"runtime.hip"}
 
 
 def test_status_strings_and_errors_without_device(vh):

@@ -441,7 +441,7 @@ static int reserve_cols(vclhip_batch_plan* plan, const vclhip_csr* A)
   if (plan->col16_dev) (void)hipFree(plan->col16_dev);
   plan->col16_dev = nullptr;
   plan->col16_cap = 0;
-  VCLHIP_HIP(hipMalloc(&plan->col16_dev, need * sizeof(uint16_t)));
+  VCLHIP_HIP(device_malloc(&plan->col16_dev, need * sizeof(uint16_t)));
   plan->col16_cap = need;
   return VCLHIP_SUCCESS;
 }
@@ -524,12 +524,12 @@ static int autotune(vclhip_batch_plan* plan, const vclhip_csr* A, const uint32_t
     if (e1) (void)hipEventDestroy(e1);
   };
   const size_t N = plan->total_rows;
-  status = hip_status(hipMalloc(&b, N * sizeof(T)), "hipMalloc");
-  if (!status) status = hip_status(hipMalloc(&x, N * sizeof(T)), "hipMalloc");
-  if (!status) status = hip_status(hipMalloc(&iters, ns * sizeof(uint32_t)), "hipMalloc");
-  if (!status) status = hip_status(hipMalloc(&conv, ns * sizeof(uint32_t)), "hipMalloc");
-  if (!status) status = hip_status(hipMalloc(&sub, ns * sizeof(uint32_t)), "hipMalloc");
-  if (!status) status = hip_status(hipMalloc(&err, ns * sizeof(double)), "hipMalloc");
+  status = hip_status(device_malloc(&b, N * sizeof(T)), "hipMalloc");
+  if (!status) status = hip_status(device_malloc(&x, N * sizeof(T)), "hipMalloc");
+  if (!status) status = hip_status(device_malloc(&iters, ns * sizeof(uint32_t)), "hipMalloc");
+  if (!status) status = hip_status(device_malloc(&conv, ns * sizeof(uint32_t)), "hipMalloc");
+  if (!status) status = hip_status(device_malloc(&sub, ns * sizeof(uint32_t)), "hipMalloc");
+  if (!status) status = hip_status(device_malloc(&err, ns * sizeof(double)), "hipMalloc");
   if (!status) status = hip_status(hipEventCreate(&e0), "hipEventCreate");
   if (!status) status = hip_status(hipEventCreate(&e1), "hipEventCreate");
   if (!status) {
@@ -587,7 +587,7 @@ static int autotune(vclhip_batch_plan* plan, const vclhip_csr* A, const uint32_t
 // blocks, else about one lane per nonzero of an average row, capped at 16.
 static int upload_lanes(vclhip_batch_plan* plan, int ti, const uint32_t* row_ptr_host)
 {
-  if (!plan->lanes_dev[ti]) VCLHIP_HIP(hipMalloc(&plan->lanes_dev[ti], plan->num_systems));
+  if (!plan->lanes_dev[ti]) VCLHIP_HIP(device_malloc(&plan->lanes_dev[ti], plan->num_systems));
   std::vector<uint8_t> lanes(plan->num_systems);
   for (uint32_t i = 0; i < plan->num_systems; ++i) {
     const uint32_t n = plan->sys_ptr[i + 1] - plan->sys_ptr[i];
@@ -701,7 +701,7 @@ int vclhip_batch_plan_create(uint32_t num_systems, const uint32_t* sys_ptr_host,
     return plan->sys_ptr[a + 1] - plan->sys_ptr[a] > plan->sys_ptr[b + 1] - plan->sys_ptr[b];
   });
   int st = hip_status(hipGetDevice(&plan->device), "hipGetDevice");
-  if (!st) st = hip_status(hipMalloc(&plan->ap_dev, std::max<size_t>(plan->total_rows, 1) * sizeof(double)), "hipMalloc");
+  if (!st) st = hip_status(device_malloc(&plan->ap_dev, std::max<size_t>(plan->total_rows, 1) * sizeof(double)), "hipMalloc");
   if (!st && row_ptr_host) {
     for (uint32_t r = 0; r < plan->total_rows && !st; ++r)
       if (row_ptr_host[r + 1] < row_ptr_host[r]) {
@@ -719,8 +719,8 @@ int vclhip_batch_plan_create(uint32_t num_systems, const uint32_t* sys_ptr_host,
       sys_blk[i + 1] = static_cast<uint32_t>(blocks.size());
     }
     blocks.push_back(plan->total_rows);
-    st = hip_status(hipMalloc(&plan->blocks_dev, blocks.size() * sizeof(uint32_t)), "hipMalloc");
-    if (!st) st = hip_status(hipMalloc(&plan->sys_blk_dev, sys_blk.size() * sizeof(uint32_t)), "hipMalloc");
+    st = hip_status(device_malloc(&plan->blocks_dev, blocks.size() * sizeof(uint32_t)), "hipMalloc");
+    if (!st) st = hip_status(device_malloc(&plan->sys_blk_dev, sys_blk.size() * sizeof(uint32_t)), "hipMalloc");
     if (!st)
       st = hip_status(hipMemcpy(plan->blocks_dev, blocks.data(), blocks.size() * sizeof(uint32_t),
                                 hipMemcpyHostToDevice), "blocks upload");
@@ -728,8 +728,8 @@ int vclhip_batch_plan_create(uint32_t num_systems, const uint32_t* sys_ptr_host,
       st = hip_status(hipMemcpy(plan->sys_blk_dev, sys_blk.data(), sys_blk.size() * sizeof(uint32_t),
                                 hipMemcpyHostToDevice), "blocks upload");
   }
-  if (!st) st = hip_status(hipMalloc(&plan->order_dev, num_systems * sizeof(uint32_t)), "hipMalloc");
-  if (!st) st = hip_status(hipMalloc(&plan->counter_dev, sizeof(uint32_t)), "hipMalloc");
+  if (!st) st = hip_status(device_malloc(&plan->order_dev, num_systems * sizeof(uint32_t)), "hipMalloc");
+  if (!st) st = hip_status(device_malloc(&plan->counter_dev, sizeof(uint32_t)), "hipMalloc");
   if (!st)
     st = hip_status(hipMemcpy(plan->order_dev, plan->order.data(), num_systems * sizeof(uint32_t),
                               hipMemcpyHostToDevice), "order upload");

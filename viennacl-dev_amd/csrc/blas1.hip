@@ -387,7 +387,7 @@ static int asum_to_host(uint32_t n, const T* x, uint32_t xs, uint32_t xi, T* res
   hipStream_t s = static_cast<hipStream_t>(stream);
   const uint32_t grid = vec_grid(n);
   void* ws = nullptr;
-  VCLHIP_HIP(hipMallocAsync(&ws, (grid + 1) * sizeof(T), s));
+  VCLHIP_HIP(stream_malloc(&ws, (grid + 1) * sizeof(T), s));
   T* part = static_cast<T*>(ws);
   hipLaunchKernelGGL(asum_partial_kernel<T>, dim3(grid), dim3(kBlock), 0, s, n, x, xs, xi, part);
   int st = check_launch("asum_partial_kernel");
@@ -411,7 +411,7 @@ static int iamax_to_host(uint32_t n, const T* x, uint32_t xs, uint32_t xi, uint3
   hipStream_t s = static_cast<hipStream_t>(stream);
   const uint32_t grid = vec_grid(n);
   void* ws = nullptr;
-  VCLHIP_HIP(hipMallocAsync(&ws, grid * (sizeof(T) + sizeof(uint32_t)) + 64, s));
+  VCLHIP_HIP(stream_malloc(&ws, grid * (sizeof(T) + sizeof(uint32_t)) + 64, s));
   T* pv = static_cast<T*>(ws);
   uint32_t* pi = reinterpret_cast<uint32_t*>(pv + grid);
   uint32_t* out = pi + grid;
@@ -463,7 +463,7 @@ static int dot_to_host(uint32_t n, const T* x, uint32_t xs, uint32_t xi, const T
   hipStream_t s = static_cast<hipStream_t>(stream);
   const uint32_t grid = vec_grid(n);
   void* ws = nullptr;
-  VCLHIP_HIP(hipMallocAsync(&ws, (grid + 1) * sizeof(A), s));
+  VCLHIP_HIP(stream_malloc(&ws, (grid + 1) * sizeof(A), s));
   A* part = static_cast<A*>(ws);
   if (xi == 1 && yi == 1)
     VCLHIP_LAUNCH_W(aligned16({x + xs, y + ys}), (dot_partial_vec_kernel<T, A, kVecW<T> >),

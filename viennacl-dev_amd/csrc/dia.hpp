@@ -434,7 +434,8 @@ struct WorkspaceDiaAlloc {
   }
 };
 
-// A quarter of the free device memory: the most an optional copy may take.
+// A quarter of the free device memory, what the workspace pool keeps counted as free: the most an
+// optional copy may take.
 inline size_t dia_memory_cap()
 {
   size_t free_b = 0, total_b = 0;
@@ -442,7 +443,7 @@ inline size_t dia_memory_cap()
     (void)hipGetLastError();
     return 0;
   }
-  return free_b / 4;
+  return (free_b + workspace_kept()) / 4;
 }
 
 }  // namespace vclhip

@@ -32,12 +32,28 @@ inline int check_launch(const char* kernel)
 int device_cu_count();
 
 // hipMallocAsync from a pool of the library's own, one per device, which keeps up to kPoolKeep freed
-// bytes for the next call (hipFreeAsync gives them back to it; the rest, and everything when an
-// allocation does not succeed otherwise, returns to the device).  The default pool keeps nothing, and
-// a solve's 132 MB operator copy then costs 85 us to map and 365 to unmap.
+// bytes for the next call (hipFreeAsync gives them back to it and the rest returns to the device).  The
+// default pool keeps nothing, and a solve's 132 MB operator copy then costs 85 us to map and 365 to
+// unmap.  What is kept must not be missing elsewhere: it goes back to the device before any allocation
+// of the library's fails (all of them go through these functions), and at the caller's request
+// (vclhip_workspace_trim).
 constexpr size_t kPoolKeep = size_t(512) << 20;
 hipError_t workspace_malloc(void** p, size_t bytes, hipStream_t s);
-void workspace_trim();  // gives back what the current device's pool keeps
+void workspace_trim();    // gives back what the current device's pool keeps
+size_t workspace_kept();  // bytes that it keeps
+
+// hipMalloc, and hipMallocAsync from the device's default pool, tried again without what the workspace
+// pool keeps.
+hipError_t device_malloc_bytes(void** p, size_t bytes);
+hipError_t stream_malloc(void** p, size_t bytes, hipStream_t s);
+template <typename U>
+inline hipError_t device_malloc(U** p, size_t bytes)
+{
+  void* v = nullptr;
+  const hipError_t e = device_malloc_bytes(&v, bytes);
+  *p = static_cast<U*>(v);
+  return e;
+}
 
 // Measurement hook (vclhip_time_next_launch): events that the next SpMV or streaming kernel
 // launched by this thread records at the kernel's own start and end.  Taking them clears them.

@@ -2593,7 +2593,7 @@ struct OwnedDiaAlloc {
   {
     void* o = nullptr;
     void* v = nullptr;
-    if (hipMalloc(&o, off_bytes) != hipSuccess || hipMalloc(&v, val_bytes) != hipSuccess) {
+    if (device_malloc(&o, off_bytes) != hipSuccess || device_malloc(&v, val_bytes) != hipSuccess) {
       (void)hipGetLastError();
       if (o) (void)hipFree(o);
       return false;

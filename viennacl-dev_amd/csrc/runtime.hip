@@ -78,6 +78,35 @@ void workspace_trim()
   if (pool && hipMemPoolTrimTo(pool, 0) != hipSuccess) (void)hipGetLastError();
 }
 
+size_t workspace_kept()
+{
+  const hipMemPool_t pool = workspace_pool();
+  uint64_t held = 0, used = 0;
+  if (!pool) return 0;
+  if (hipMemPoolGetAttribute(pool, hipMemPoolAttrReservedMemCurrent, &held) != hipSuccess ||
+      hipMemPoolGetAttribute(pool, hipMemPoolAttrUsedMemCurrent, &used) != hipSuccess) {
+    (void)hipGetLastError();
+    return 0;
+  }
+  return held > used ? static_cast<size_t>(held - used) : 0;
+}
+
+hipError_t device_malloc_bytes(void** p, size_t bytes)
+{
+  if (hipMalloc(p, bytes) == hipSuccess) return hipSuccess;
+  (void)hipGetLastError();
+  workspace_trim();
+  return hipMalloc(p, bytes);
+}
+
+hipError_t stream_malloc(void** p, size_t bytes, hipStream_t s)
+{
+  if (hipMallocAsync(p, bytes, s) == hipSuccess) return hipSuccess;
+  (void)hipGetLastError();
+  workspace_trim();
+  return hipMallocAsync(p, bytes, s);
+}
+
 __global__ __launch_bounds__(kBlock) void fill_bytes_kernel(uint8_t* __restrict__ p, size_t bytes)
 {
   // 16-byte stores over the aligned body, byte stores for the head and tail
@@ -163,10 +192,13 @@ int vclhip_malloc(void** ptr, size_t bytes)
   if (!ptr) return vclhip::invalid("ptr is NULL");
   *ptr = nullptr;
   if (bytes == 0) return VCLHIP_SUCCESS;
-  if (hipMalloc(ptr, bytes) == hipSuccess) return VCLHIP_SUCCESS;
-  (void)hipGetLastError();
-  vclhip::workspace_trim();  // what the solvers' pool keeps may be what is missing
-  VCLHIP_HIP(hipMalloc(ptr, bytes));
+  VCLHIP_HIP(vclhip::device_malloc_bytes(ptr, bytes));
+  return VCLHIP_SUCCESS;
+}
+
+int vclhip_workspace_trim(void)
+{
+  vclhip::workspace_trim();
   return VCLHIP_SUCCESS;
 }
 

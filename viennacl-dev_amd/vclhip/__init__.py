@@ -30,6 +30,11 @@ def device_count():
     return c.value
 
 
+def workspace_trim():
+    """Gives back to the device what the solvers keep of it for the next solve (at most 512 MB)."""
+    call("vclhip_workspace_trim")
+
+
 class Stream:
     """A non-blocking HIP stream owned by the caller (None = null stream)."""
 

@@ -102,6 +102,7 @@ _SIGS = {
     "vclhip_device_info": (i32, [i32, C.c_char_p, sz, P(sz), P(i32), P(i32), P(i32)]),
     "vclhip_malloc": (i32, [P(vp), sz]),
     "vclhip_free": (i32, [vp]),
+    "vclhip_workspace_trim": (i32, []),
     "vclhip_memcpy_h2d": (i32, [vp, vp, sz, vp]),
     "vclhip_memcpy_d2h": (i32, [vp, vp, sz, vp]),
     "vclhip_memcpy_d2d": (i32, [vp, vp, sz, vp]),
