@@ -5,6 +5,7 @@ stopping quantity below the tag tolerance, and the FP64 true residual ||b - A x|
 Element-wise updates are bit-exact against the reference (no contraction, same expressions);
 inner products differ only in summation order.
 """
+import contextlib
 import ctypes as C
 import pathlib
 
@@ -18,6 +19,19 @@ GOLDEN = pathlib.Path(__file__).resolve().parent / "golden"
 
 def load(name):
     return dict(np.load(GOLDEN / f"{name}.npz", allow_pickle=False))
+
+
+@contextlib.contextmanager
+def on_chip(vh, wanted):
+    """CG solves of this thread that run all iterations in one launch (wanted), or that leave that mode out."""
+    off, last = vh.lib().onchip_cg_off, vh.lib().onchip_cg_last
+    off(0 if wanted else 1)
+    last()
+    try:
+        yield
+    finally:
+        off(0)
+    assert last() == (1 if wanted else 0)
 
 
 def close_sum(a, b, scale):
@@ -522,7 +536,8 @@ def test_cg_one_kernel_per_iteration_equals_two(dev, vh, oracle, case):
     for variant in (0, 1):
         db, dx = vh.DeviceArray.from_numpy(b), vh.DeviceArray.zeros(n, np.float64)
         hist = np.zeros(kw["max_iters"])
-        res = vh.cg(A, db, dx, precond=pc, variant=variant, history=hist, **kw)
+        with on_chip(vh, False):
+            res = vh.cg(A, db, dx, precond=pc, variant=variant, history=hist, **kw)
         out.append((dx.to_numpy(), res, hist))
     (xf, rf, hf), (xc, rc, hc) = out
     print(f"{case}: {rf.iters} iterations, kernels per iteration {rf.kernels_per_iter} / {rc.kernels_per_iter}")
@@ -568,7 +583,8 @@ def test_cg_fused_mode_only_below_its_partial_read_bound(dev, vh, case):
     out = []
     for variant in (0, 1):
         db, dx = vh.DeviceArray.from_numpy(b), vh.DeviceArray.zeros(n, np.float64)
-        res = vh.cg(A, db, dx, tol=1e-8, max_iters=3000, variant=variant)
+        with on_chip(vh, False):
+            res = vh.cg(A, db, dx, tol=1e-8, max_iters=3000, variant=variant)
         out.append((dx.to_numpy(), res))
     (x0, r0), (x1, r1) = out
     assert r0.operator_used == vh.USED_DIA and r0.kernels_per_iter == want and r1.kernels_per_iter == 2
@@ -671,11 +687,13 @@ def test_solvers_refuse_vectors_of_another_precision_or_size(dev, vh):
         vh.mixed_cg(A64, b32, x32)
 
 
-def test_concurrent_solves_on_two_streams_match_sequential(dev, vh):
+@pytest.mark.parametrize("one_launch", [False, True])
+def test_concurrent_solves_on_two_streams_match_sequential(dev, vh, one_launch):
     """The solvers keep their state per call (workspace, scalar record, partial sums on the caller's
     stream), so solves issued from two host threads on two streams run concurrently and give what
     they give one after the other, bit for bit: CG and BiCGStab, a small system (one kernel per CG
-    iteration) beside a larger one (three), each thread repeating its solves."""
+    iteration) beside a larger one (three), each thread repeating its solves; and with the mode that
+    runs a whole CG in one launch, which one of the two threads at a time may take."""
     import threading
 
     systems = [vh.fdm_laplace_2d(200, 200), vh.laplace_3d(48)]
@@ -704,6 +722,7 @@ def test_concurrent_solves_on_two_streams_match_sequential(dev, vh):
     errors = []
 
     def worker(i):
+        vh.lib().onchip_cg_off(0 if one_launch else 1)  # for this thread
         try:
             for r in range(reps):
                 got[i].append(run(i, r, streams[i].handle))
@@ -742,28 +761,32 @@ def tridiag(n):
 @pytest.mark.parametrize("n", [1, 2, 5, 63, 64, 65, 257])
 def test_tiny_systems_every_launch_mode(dev, vh, n):
     """Systems of 1 to 257 rows (partial packs, chunks smaller than a workgroup, grids at their
-    minimum of 8 workgroups) in every launch mode: CG in one and two kernels per iteration and
-    BiCGStab in four and six give the same x bit for bit and solve the system; a NaN in b ends at
+    minimum of 8 workgroups) in every launch mode: CG in one launch, in one and in two kernels per
+    iteration and BiCGStab in four and six give the same x bit for bit and solve the system; a NaN in b ends at
     the iteration cap in every mode.  When s vanishes exactly (a one- or two-row system), the
     pipelined BiCGStab's omega is 0/0, as in the reference (bicgstab.hpp:193-195); there only the
     agreement of the modes is checked."""
     rp, col, val = tridiag(n)
     A = vh.CsrMatrix(rp, col, val)
     b = vh.random_uniform(3, n)
-    for kind, modes in (("cg", (0, 1)), ("bicgstab", (0, 1))):
+    # two rows: the padding of a DIA copy, which the one launch needs, would be half of the entries
+    for kind, modes in (("cg", ((0, n != 2), (0, False), (1, False))), ("bicgstab", ((0, False), (1, False)))):
         exact_breakdown = kind == "bicgstab" and n <= 2
         xs = []
-        for variant in modes:
-            x, res = solve(vh, kind, A, b, tol=1e-10, max_iters=4 * n + 20, variant=variant)
+        for variant, one_launch in modes:
+            with on_chip(vh, one_launch):
+                x, res = solve(vh, kind, A, b, tol=1e-10, max_iters=4 * n + 20, variant=variant)
             assert res.converged or exact_breakdown, (kind, variant, res.iters)
             xs.append((x, res.iters))
-        assert np.array_equal(xs[0][0], xs[1][0], equal_nan=True) and xs[0][1] == xs[1][1], kind
+        for x, iters in xs[1:]:
+            assert np.array_equal(xs[0][0], x, equal_nan=True) and xs[0][1] == iters, kind
         if not exact_breakdown:
             assert true_relres(rp, col, val, xs[0][0], b) < 1e-8
         bn = b.copy()
         bn[n // 2] = np.nan
-        for variant in modes:
-            _, res = solve(vh, kind, A, bn, tol=1e-10, max_iters=30, variant=variant)
+        for variant, one_launch in modes:
+            with on_chip(vh, one_launch):
+                _, res = solve(vh, kind, A, bn, tol=1e-10, max_iters=30, variant=variant)
             assert res.iters == 30 and not res.converged, (kind, variant)
 
 
@@ -784,17 +807,18 @@ def abs_tol_oracle(oracle, H, key, b, abs_tol, jacobi_diag):
     return _ABS_ORACLE[key]
 
 
-@pytest.mark.parametrize("case", ["fdm_256_fused", "fdm_256_two_kernels", "lap3d_96_dia", "lap3d_96_as_given",
-                                  "lap3d_40_sell"])
+@pytest.mark.parametrize("case", ["fdm_256_one_launch", "fdm_256_fused", "fdm_256_two_kernels", "lap3d_96_one_launch",
+                                  "lap3d_96_dia", "lap3d_96_as_given", "lap3d_40_sell"])
 def test_absolute_tolerance_stop_vs_oracle(dev, vh, oracle, case):
     """abs_tolerance(): CG stops when |<r,r>| < abs_tol^2 (cg.hpp:176, classic form :309) and
     BiCGStab when ||r|| < abs_tol (bicgstab.hpp:198, :465), whichever of the two tests comes first.
     With a relative tolerance out of reach (1e-15) the absolute one ends the solve at the oracle's
-    iteration count in every launch mode (one fused kernel, two, three on the 96^3 operator; DIA
+    iteration count in every launch mode (one launch, one fused kernel an iteration, two, three on the 96^3 operator; DIA
     copy, CSR as given, SELL-64), and ||b|| below abs_tol returns x = 0 at once (cg.hpp:151,
     bicgstab.hpp:140)."""
-    m, kw = {"fdm_256_fused": (256, {}), "fdm_256_two_kernels": (256, {"variant": 1}),
-             "lap3d_96_dia": (96, {}), "lap3d_96_as_given": (96, {"operator_format": vh.OPERATOR_AS_GIVEN}),
+    m, kw = {"fdm_256_one_launch": (256, {}), "fdm_256_fused": (256, {}), "fdm_256_two_kernels": (256, {"variant": 1}),
+             "lap3d_96_one_launch": (96, {}), "lap3d_96_dia": (96, {}),
+             "lap3d_96_as_given": (96, {"operator_format": vh.OPERATOR_AS_GIVEN}),
              "lap3d_40_sell": (40, {})}[case]
     rp, col, val = vh.fdm_laplace_2d(m, m) if case.startswith("fdm") else vh.laplace_3d(m)
     n = rp.size - 1
@@ -808,11 +832,15 @@ def test_absolute_tolerance_stop_vs_oracle(dev, vh, oracle, case):
     abs_tol = 1e-5 * nb
     diag = None if sell else oracle.row_info(rp, col, val, 3)
     cg_it, jac_it, env, bicg_hist = abs_tol_oracle(oracle, H, (case.split("_")[0], m, sell), b, abs_tol, diag)
-    x, res = solve(vh, "cg", A, b, tol=1e-15, abs_tol=abs_tol, max_iters=5000, **kw)
+    one_launch = case.endswith("one_launch")
+    with on_chip(vh, one_launch):
+        x, res = solve(vh, "cg", A, b, tol=1e-15, abs_tol=abs_tol, max_iters=5000, **kw)
     assert res.converged and iters_close(res.iters, cg_it), (res.iters, cg_it)
     assert true_relres(rp, col, val, x, b) < 1.1e-5
     if not sell:
-        _, res = solve(vh, "cg", A, b, precond=vh.PRECOND_JACOBI, tol=1e-15, abs_tol=abs_tol, max_iters=5000, **kw)
+        with on_chip(vh, one_launch):
+            _, res = solve(vh, "cg", A, b, precond=vh.PRECOND_JACOBI, tol=1e-15, abs_tol=abs_tol, max_iters=5000,
+                           **kw)
         assert res.converged and iters_close(res.iters, jac_it), (res.iters, jac_it)
     # BiCGStab's residual is jagged at this level: the oracle's own count moves by up to 13% with
     # the summation order (114-129 on the 96^3 case), and the reference's, whose OpenMP reductions

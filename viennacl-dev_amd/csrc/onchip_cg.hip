@@ -55,10 +55,11 @@
 
 namespace vclhip {
 
-// Hooks of the tests (onchip_cg_wait_limit, onchip_cg_last and onchip_cg_plan, not part of the API), per
-// thread: the wait limit in microseconds (below zero: the usual ones), and whether the last CG solve ran
-// here (1), gave up (2) or neither (0).
+// Hooks of the tests (onchip_cg_wait_limit, onchip_cg_off, onchip_cg_last and onchip_cg_plan, not part of
+// the API), per thread: the wait limit in microseconds (below zero: the usual ones), whether solves leave
+// this mode out, and whether the last CG solve ran here (1), gave up (2) or neither (0).
 static thread_local double t_wait_us = -1;
+static thread_local bool t_off = false;
 static thread_local int t_on_chip = 0;
 
 namespace {
@@ -969,7 +970,7 @@ int onchip_cg(const OnchipCg<T>& c, Workspace& ws, hipStream_t s, KState* fin, O
   *outcome = Onchip::kNo;
   t_on_chip = 0;
   OcPlan<T> pl;
-  if (!oc_plan(c, static_cast<uint32_t>(device_cu_count()), pl)) return VCLHIP_SUCCESS;
+  if (t_off || !oc_plan(c, static_cast<uint32_t>(device_cu_count()), pl)) return VCLHIP_SUCCESS;
   int dev = 0;
   VCLHIP_HIP(hipGetDevice(&dev));
   if (dev < 0 || dev >= 64) return VCLHIP_SUCCESS;
@@ -1063,6 +1064,12 @@ extern "C" {
 int onchip_cg_wait_limit(double microseconds)
 {
   vclhip::t_wait_us = microseconds;
+  return VCLHIP_SUCCESS;
+}
+
+int onchip_cg_off(int off)
+{
+  vclhip::t_off = off != 0;
   return VCLHIP_SUCCESS;
 }
 
