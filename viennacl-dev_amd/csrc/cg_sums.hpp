@@ -20,10 +20,12 @@ constexpr uint32_t kCgVecRows = 1u << 18;  // rows of all owners' vector chunks 
 constexpr uint32_t kCgVecPerOwner = 8;     // vector chunks per owner at most
 static_assert(kCgProdMax <= kMaxPartials && kOwners * kCgVecPerOwner <= kMaxPartials && kMaxPartials <= 4096, "partial sums");
 
-// [begin, end) of part i of `parts` near-equal contiguous parts of `total` items.
+// [begin, end) of part i of `parts` (at most kCgProdMax) near-equal contiguous parts of `total` items.
+constexpr uint32_t kPartShort = 1u << 20;
+static_assert(static_cast<uint64_t>(kPartShort) * kCgProdMax < 1ull << 32 && kOwners <= kCgProdMax, "products of 32 bits");
 __host__ __device__ inline void part_range(uint32_t total, uint32_t i, uint32_t parts, uint32_t& begin, uint32_t& end)
 {
-  if (total <= 1u << 20) {  // at most 4096 parts: 32 bits hold the product, and its division is the shorter one
+  if (total <= kPartShort) {  // 32 bits hold the product, and its division is the shorter one
     begin = total * i / parts;
     end = total * (i + 1) / parts;
   } else {

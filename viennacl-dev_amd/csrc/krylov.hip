@@ -37,8 +37,11 @@ constexpr uint64_t kCompactPartialReads = 1ull << 20;
 // (450^2).
 constexpr uint64_t kFusedPartialReads = 1ull << 19;
 // BiCGStab with the reference's Jacobi recurrences: alpha and omega inside the vector kernels up to so
-// many partials read by all workgroups together, of the larger of the two sums (400 000 power-law rows,
-// 1.6 M reads: 52 us an iteration for 56; a scalar kernel takes 3.7 us and a launch).
+// many partials read by all workgroups together, of the larger of the two sums.  A scalar kernel and its
+// launch take about 3.7 us; an iteration with it and without (us): power-law rows, 200 K (0.4 M reads)
+// 43.7 and 40.2, 400 K (1.2 M) 64.8 and 61.6, 500 K (1.9 M) 75.8 and 72.1; 80^3 convection (2.0 M) 38.4
+// and 36.2.  The bound is where the gain was still all of it: past it 95.6 and 92.3 at 600 K rows (2.4 M),
+// 127.2 and 126.7 at 800 K (3.2 M), 159.9 and 157.1 at 1 M (4.0 M), 70.5 and 66.9 for 110^3 (5.3 M).
 constexpr uint64_t kClassicPartialReads = 1ull << 21;
 
 // ------------------------------------------------------------------ epilogues

@@ -15,7 +15,7 @@
 //       sums: one exchange per iteration.  Up to two rows a lane (n <= 2^19);
 //     halo:  p of the own rows is stored after the update, neighbours are told by a flag, and the
 //       reached rows are read from memory: a second, neighbours-only wait per iteration (about 1 us),
-//       but no ghost state.  With more than two rows a lane the ghosts' registers spill (100^3: 24 us
+//       for as many workgroups on each side as own reached rows (oc_reach), but no ghost state.  With more than two rows a lane the ghosts' registers spill (100^3: 24 us
 //       an iteration as ghost, 11 as halo; Jacobi on 97 x 83 x 71: 30 and 20).
 // From 128 workgroups on, the first of each XCD adds up its XCD's sums and all others read those eight:
 // 256 workgroups that poll 256 lines hold each other up (exchange at 64^3 3.5 us, 2.4 in two steps;
@@ -28,7 +28,7 @@
 // diagonal has one value (the constant-coefficient Laplacians), as packed 4-bit codes into value
 // tables in LDS, or as stored: as many diagonals as fit in LDS, the others read again in every iteration
 // (Jacobi-CG on 97 x 83 x 71, whose 32 MB of values come to just the L2s' size: 20 us an iteration with
-// all of them read, 12 with six of seven diagonals in LDS).
+// all of them read, 12 with six of seven diagonals in LDS, 9.5 since the sums meet per XCD first).
 //
 // What bounds it: 256^2 runs 3.9 us an iteration, of which the exchange of the sums takes 1.7 and the
 // workgroup's own sums 0.6 (7.4 us with one launch per iteration); 128^3 runs 14 us (47 us with three):
@@ -36,8 +36,8 @@
 // XCDs' edges, whose far rows come from further away.
 //
 // The mixed solver runs its FP32 inner iterations between two FP64 corrections the same way, up to 16
-// rows a lane: 160^3 variable coefficients 36 us an iteration (55 us with three launches), of which the
-// FP32 values, 115 MB read from the Infinity Cache, are the larger part.
+// rows a lane: 160^3 variable coefficients 29 us an iteration (51 us with three launches), of which the
+// FP32 values, 115 MB read from the Infinity Cache, are the larger part (19 us at 6 TB/s).
 //
 // Every sum is formed in the order of the kernel-per-step modes (cg_sums.hpp), so the results are
 // theirs bit for bit.
