@@ -1,5 +1,6 @@
 """CG with all iterations in one launch (onchip_cg.hip) against the kernel-per-step modes, bit for bit."""
 import ctypes
+import threading
 
 import numpy as np
 import pytest
@@ -147,6 +148,44 @@ def test_workgroups_that_start_after_others_gave_up(dev, vh, case):
             assert mode == GAVE_UP and np.array_equal(x, want)
     finally:
         limit(-1.0)
+
+
+@pytest.mark.parametrize("case", ["whole_device", "quarters", "mixed_sizes"])
+def test_solves_of_several_threads_take_turns(dev, vh, case):
+    """Solves of host threads on streams of their own: each waits for the compute units it needs and runs on
+    chip (none is left to the launched modes, beside which it would hardly progress), one after the other
+    or together where they fit, over several launches too; all give what they give alone."""
+    whole, quarter = (300001, [1, 547], 0), (60001, [1, 245], 0)
+    systems = {"whole_device": [whole, whole], "quarters": [quarter] * 6, "mixed_sizes": [whole, quarter, quarter]}[case]
+    made = {s[0]: band(*s, seed=s[0]) for s in systems}
+    reps, kw = 6, dict(tol=0.0, max_iters=5000 if case == "mixed_sizes" else 300)
+    mats = [vh.CsrMatrix(*made[s[0]]) for s in systems]
+    arrays = [(vh.DeviceArray.from_numpy(vh.random_uniform(7, s[0])), vh.DeviceArray.zeros(s[0], np.float64)) for s in systems]
+    want = []
+    for A, (b, x) in zip(mats, arrays):
+        vh.cg(A, b, x, **kw)
+        want.append(x.to_numpy())
+    streams = [vh.Stream() for _ in systems]
+    vh.call("vclhip_device_synchronize")
+    modes, got = [[] for _ in systems], [None] * len(systems)
+
+    def work(i):
+        for _ in range(reps):
+            vh.lib().onchip_cg_last()
+            vh.cg(mats[i], *arrays[i], stream=streams[i].handle, **kw)
+            modes[i].append(vh.lib().onchip_cg_last())
+        got[i] = arrays[i][1].to_numpy(streams[i].handle)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(systems))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(timeout=60)
+    assert not any(t.is_alive() for t in threads)
+    assert all(m == [RAN] * reps for m in modes), modes
+    assert all(np.array_equal(g, w, equal_nan=True) for g, w in zip(got, want))
+    for s in streams:
+        s.close()
 
 
 @pytest.mark.parametrize("precond", [0, 1])

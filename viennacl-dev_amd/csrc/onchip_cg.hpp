@@ -30,8 +30,8 @@ struct OnchipCg {
 
 enum class Onchip { kNo, kDone, kAborted };
 
-// Runs the iterations to the end if the system fits.  kNo: it does not (or another solve of this
-// process holds the device's on-chip slot): nothing was launched and the solve stands as before.
+// Runs the iterations to the end if the system fits; where other threads' solves hold the CUs it waits for
+// its turn.  kNo: it does not fit: nothing was launched and the solve stands as before.
 // kAborted: the workgroups could not all run at once within the wait limit; the vectors and *st are
 // then undefined and the caller starts over with the other modes.  kDone: x is written and *fin is the final state.
 template <typename T>
