@@ -448,7 +448,10 @@ typedef struct vclhip_solver_params {
                                         results are the same bit for bit.
                                         CG: 0 = automatic (a system on a DIA operator whose vectors fit
                                         the compute units' registers runs all iterations in one
-                                        kernel, a small one otherwise one kernel per iteration),
+                                        kernel, a small one otherwise one kernel per iteration;
+                                        that one kernel holds up to all compute units for as long
+                                        as it runs, at most 4096 iterations, and kernels of other
+                                        streams wait for its end),
                                         1 = at least two kernels per iteration; the results are the
                                         same bit for bit */
   double* history_host;              /* optional: per-iteration convergence quantity (may be NULL) */

@@ -188,6 +188,39 @@ def test_solves_of_several_threads_take_turns(dev, vh, case):
         s.close()
 
 
+def test_leaves_the_device_to_another_threads_launched_solve(dev, vh):
+    """Beside a BiCGStab solve of another thread a CG that would take the whole device runs launched, one
+    that takes a quarter of it on chip; both on chip again afterwards.  The results are the same."""
+    rp, col, val = vh.convection_diffusion(40, 40, 40)
+    C, cb, cx = vh.CsrMatrix(rp, col, val), vh.DeviceArray.from_numpy(vh.random_uniform(2, 64000)), vh.DeviceArray.zeros(64000, np.float64)
+    solves = [(vh.CsrMatrix(*band(n, o, 0)), vh.random_uniform(3, n), mode)
+              for n, o, mode in ((300001, [1, 547], NOT_RUN), (60001, [1, 245], RAN))]
+    kw, stream = dict(tol=1e-9, max_iters=400), vh.Stream()
+    want = [run(vh, A, b, np.float64, **kw) for A, b, _ in solves]
+    vh.call("vclhip_device_synchronize")
+    beside, stop = threading.Event(), threading.Event()
+
+    @vh.MONITOR
+    def going_on(x, rel, user):
+        beside.set()
+        return 1 if stop.is_set() else 0
+
+    t = threading.Thread(target=lambda: vh.bicgstab(C, cb, cx, tol=0.0, max_iters=1000000, monitor=going_on, stream=stream.handle))
+    t.start()
+    try:
+        assert beside.wait(30)
+        got = [run(vh, A, b, np.float64, **kw) for A, b, _ in solves]
+    finally:
+        stop.set()
+        t.join(timeout=60)
+    assert not t.is_alive()
+    for (x, _, h, mode), (x0, _, h0, mode0), (_, _, expected) in zip(got, want, solves):
+        assert mode0 == RAN and mode == expected and np.array_equal(x, x0) and np.array_equal(h, h0)
+    for A, b, _ in solves:
+        assert run(vh, A, b, np.float64, **kw)[3] == RAN
+    stream.close()
+
+
 @pytest.mark.parametrize("precond", [0, 1])
 def test_solution_over_the_right_hand_side(dev, vh, precond):
     """b and x in one array: the launched modes read b before they write x.  The one-launch solve gives the

@@ -29,6 +29,7 @@
 #include <vector>
 
 #include "internal.hpp"
+#include "onchip_cg.hpp"
 #include "solver.hpp"
 #include "dia.hpp"
 #include "spmv_kernels.hpp"
@@ -545,6 +546,7 @@ int gmres_solve(const M* Ain, const T* b, T* x, const vclhip_solver_params* P, v
   if (max_restarts > 0 && max_restarts * K == P->max_iters) max_restarts -= 1;
   const uint32_t max_cycles = max_restarts + 1;
 
+  const LaunchedSolve launched;
   Workspace ws(s);
   int used_dia = 0;
   VCLHIP_TRY(dia_operator(op, ws, s, P, &used_dia));

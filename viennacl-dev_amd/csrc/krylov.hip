@@ -1505,6 +1505,8 @@ static int cg_solve(const M* Ain, const T* b, T* x, int precond, const vclhip_so
     VCLHIP_TRY(onchip_cg<T>({n, op.dia, jac, v2, x, r, p, Ap, d, st, nullptr}, ws, s, &fin, &on_chip));
     if (on_chip == Onchip::kAborted) VCLHIP_TRY(start());
   }
+  std::optional<LaunchedSolve> launched;
+  if (on_chip == Onchip::kNo || on_chip == Onchip::kAborted) launched.emplace();
   if (on_chip == Onchip::kDone) {
     // x and fin are there
   } else if (compact) {
@@ -1551,6 +1553,7 @@ static int bicgstab_solve(const M* Ain, const T* b, T* x, int precond, const vcl
   hipStream_t s = ss.get();
   const uint32_t n = op.n;
   const bool jac = precond == VCLHIP_PRECOND_JACOBI;
+  const LaunchedSolve launched;
   Workspace ws(s);
   int used_dia = 0;
   VCLHIP_TRY(dia_operator(op, ws, s, P, &used_dia));
@@ -2446,10 +2449,13 @@ static int mixed_cg_solve(const M* A, const float* values32, const double* b, do
     VCLHIP_TRY(onchip_cg<float>({n, op32.dia, false, true, x32, r32, p32, Ap32, nullptr, st, tail}, ws, s, &fin, &on_chip));
     if (on_chip == Onchip::kAborted) VCLHIP_TRY(start());
   }
-  if (on_chip != Onchip::kDone)
+  if (on_chip != Onchip::kDone) {
+    std::optional<LaunchedSolve> launched;
+    if (on_chip != Onchip::kDeferred) launched.emplace();
     VCLHIP_TRY(run_iterations(
         s, st, 0u, P->max_iters, P, x, launch_iter, [](uint32_t) { return false; }, [](uint32_t) { return 0; }, fin,
         false, tail));
+  }
   R->iters = fin.iter;
   R->error = fin.nrs > 0 ? std::sqrt(fin.res / fin.nrs) : 0.0;
   R->restarts = fin.updates;

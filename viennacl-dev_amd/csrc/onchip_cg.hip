@@ -852,6 +852,21 @@ __global__ __launch_bounds__(kOcThreads) void onchip_cg_kernel(OcArgs<T> a)
 
 // ------------------------------------------------------------------ host side
 
+// The solves that run on a device, for those of other host threads.
+struct OcDevice {
+  std::mutex mu;
+  std::condition_variable cv;
+  uint32_t used = 0;               // CUs of the on-chip launches that run
+  uint32_t launched = 0;           // solves that run by launches of their own (LaunchedSolve)
+  uint64_t tickets = 0, turn = 0;  // of the on-chip launches: given out, and whose turn it is
+};
+constexpr int kOcDevices = 64;
+OcDevice* oc_device(int dev)
+{
+  static OcDevice* const d = new OcDevice[kOcDevices];  // never freed: threads may still wait when the process ends
+  return dev >= 0 && dev < kOcDevices ? d + dev : nullptr;
+}
+
 // A solve's share of its device's CUs while a launch of its runs.  Solves of several host threads whose
 // workgroups fit the device together run together; the others wait, in the order in which they came, and
 // a solve of more than one launch queues again between them.  A solve that took the launched modes
@@ -859,10 +874,18 @@ __global__ __launch_bounds__(kOcThreads) void onchip_cg_kernel(OcArgs<T> a)
 // Jacobi-CG on 97 x 83 x 71 one got 2.5 solves a second and the other 130 (41.6 each if both are launched).
 class OcTurn {
  public:
-  OcTurn(int dev, uint32_t cus, uint32_t want) : d_(devices()[dev]), cus_(cus), want_(want) {}
+  OcTurn(OcDevice* d, uint32_t cus, uint32_t want) : d_(*d), cus_(cus), want_(want) {}
   ~OcTurn() { give(); }
   OcTurn(const OcTurn&) = delete;
   OcTurn& operator=(const OcTurn&) = delete;
+  // Whether a first launch should be left out: it would take most of the device from a solve that another
+  // thread runs by launches (BiCGStab on 70 x 66 x 61 beside Jacobi-CG on 97 x 83 x 71 got 20 solves a second,
+  // and 157 with both launched; a quarter of the CUs leaves it 144).
+  bool in_the_way() const
+  {
+    std::lock_guard<std::mutex> lock(d_.mu);
+    return d_.launched > 0 && want_ > cus_ / 4;
+  }
   void take()
   {
     std::unique_lock<std::mutex> lock(d_.mu);
@@ -881,21 +904,9 @@ class OcTurn {
     held_ = false;
     d_.cv.notify_all();
   }
-  static constexpr int kDevices = 64;
 
  private:
-  struct Device {
-    std::mutex mu;
-    std::condition_variable cv;
-    uint32_t used = 0;              // CUs of the launches that run
-    uint64_t tickets = 0, turn = 0;  // given out; whose turn it is
-  };
-  static Device* devices()
-  {
-    static Device* const d = new Device[kDevices];  // never freed: threads may still wait when the process ends
-    return d;
-  }
-  Device& d_;
+  OcDevice& d_;
   const uint32_t cus_, want_;
   bool held_ = false;
 };
@@ -1010,6 +1021,23 @@ bool oc_plan(const OnchipCg<T>& c, uint32_t cus, OcPlan<T>& pl)
 
 }  // namespace
 
+LaunchedSolve::LaunchedSolve()
+{
+  if (hipGetDevice(&dev_) != hipSuccess || !oc_device(dev_)) {
+    dev_ = -1;
+    return;
+  }
+  std::lock_guard<std::mutex> lock(oc_device(dev_)->mu);
+  ++oc_device(dev_)->launched;
+}
+
+LaunchedSolve::~LaunchedSolve()
+{
+  if (dev_ < 0) return;
+  std::lock_guard<std::mutex> lock(oc_device(dev_)->mu);
+  --oc_device(dev_)->launched;
+}
+
 template <typename T>
 int onchip_cg(const OnchipCg<T>& c, Workspace& ws, hipStream_t s, KState* fin, Onchip* outcome)
 {
@@ -1020,7 +1048,13 @@ int onchip_cg(const OnchipCg<T>& c, Workspace& ws, hipStream_t s, KState* fin, O
   if (t_off || !oc_plan(c, cus, pl)) return VCLHIP_SUCCESS;
   int dev = 0;
   VCLHIP_HIP(hipGetDevice(&dev));
-  if (dev < 0 || dev >= OcTurn::kDevices) return VCLHIP_SUCCESS;
+  OcDevice* const device = oc_device(dev);
+  if (!device) return VCLHIP_SUCCESS;
+  OcTurn turn(device, cus, pl.nwg);
+  if (turn.in_the_way()) {
+    *outcome = Onchip::kDeferred;
+    return VCLHIP_SUCCESS;
+  }
   VCLHIP_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(pl.kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                  static_cast<int>(pl.lds)));
   int per_cu = 0;
@@ -1064,7 +1098,6 @@ int onchip_cg(const OnchipCg<T>& c, Workspace& ws, hipStream_t s, KState* fin, O
   a.wait_first = wait_ticks(true);
   a.wait = wait_ticks(false);
   // (what is still to run in front of the launch is the setup's few kernels: start() waited for the stream)
-  OcTurn turn(dev, cus, pl.nwg);
   do {
     turn.take();
     hipLaunchKernelGGL(pl.kernel, dim3(pl.nwg), dim3(kOcThreads), pl.lds, s, a);

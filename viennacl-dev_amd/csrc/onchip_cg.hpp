@@ -3,6 +3,7 @@
 #pragma once
 
 #include <functional>
+#include <optional>
 
 #include "krylov_state.hpp"
 #include "solver.hpp"
@@ -28,10 +29,25 @@ struct OnchipCg {
   std::function<int()> after;
 };
 
-enum class Onchip { kNo, kDone, kAborted };
+enum class Onchip { kNo, kDeferred, kDone, kAborted };
+
+// For as long as it lives, a solve that runs by launches of its own: another thread's solve then leaves
+// the one-launch mode out if that took more than a quarter of the device.  Not made for a solve that was
+// left out itself (two of them would keep each other from it).
+class LaunchedSolve {
+ public:
+  LaunchedSolve();
+  ~LaunchedSolve();
+  LaunchedSolve(const LaunchedSolve&) = delete;
+  LaunchedSolve& operator=(const LaunchedSolve&) = delete;
+
+ private:
+  int dev_ = -1;
+};
 
 // Runs the iterations to the end if the system fits; where other threads' solves hold the CUs it waits for
-// its turn.  kNo: it does not fit: nothing was launched and the solve stands as before.
+// its turn.  kNo: it does not fit; kDeferred: another thread's LaunchedSolve needs the device.  Nothing was
+// launched then and the solve stands as before.
 // kAborted: the workgroups could not all run at once within the wait limit; the vectors and *st are
 // then undefined and the caller starts over with the other modes.  kDone: x is written and *fin is the final state.
 template <typename T>
